@@ -207,8 +207,9 @@ __global__ __launch_bounds__(kThreads) void k_grid_finish(GridReduce g, uint32_t
 }
 
 // grids above this many workgroups defer their reduction to k_grid_finish (below it the
-// in-kernel finish costs less than the extra launch)
-constexpr uint64_t kDeferGrid = 512;
+// in-kernel finish costs less than the extra launch: a defect with its norm on 396 workgroups
+// 8.6 us deferred against 11.7, on 129 workgroups 7.6 against 6.6)
+constexpr uint64_t kDeferGrid = 256;
 
 __host__ inline GridReduce reduce_for_grid(GridReduce g, uint64_t grid)
 {

@@ -72,6 +72,18 @@ struct EpiPre<E, std::void_t<typename E::Pre>>
   static constexpr bool on = true;
 };
 
+// EpiCentre<E>::on: E::pre takes the row's entry of x where the caller holds it
+template<class E, typename DT, class = void>
+struct EpiCentre
+{
+  static constexpr bool on = false;
+};
+template<class E, typename DT>
+struct EpiCentre<E, DT, std::void_t<decltype(std::declval<const E&>().pre(uint64_t(0), DT(0)))>>
+{
+  static constexpr bool on = true;
+};
+
 // ---------------------------------------------------------------------------
 // CSR row-block kernel with a fused epilogue.
 //   Epi::row(row, sum, acc0, acc1) is called once per row by its lane.
@@ -152,6 +164,9 @@ __global__ __launch_bounds__(kThreads) void k_csr_rows(const DT* __restrict__ va
   grid_reduce_finish(gr, acc0, acc1);
 }
 
+// Every epilogue: filtered(pre) says that the row's result does not depend on its sum (the
+// unit filter sets the value that the sum goes into to zero).
+//
 // r = a*sum + b*y  (y not read when |b| < eps)          [arch/apply_generic.hpp:30-66]
 template<typename DT>
 struct EpiApply
@@ -167,6 +182,7 @@ struct EpiApply
     DT yv;
   };
   __device__ __forceinline__ Pre pre(uint64_t i) const { return Pre{bzero ? DT(0) : y[i]}; }
+  __device__ __forceinline__ bool filtered(const Pre&) const { return false; }
   __device__ __forceinline__ void row(uint64_t i, DT sum, const Pre& p, double&, double&) const
   {
     r[i] = dfma(sum, a, b * p.yv);
@@ -214,6 +230,7 @@ struct EpiMasked
   {
     return Pre{dot ? dotw[i] : DT(0), first.load(i), is_masked(mask, i)};
   }
+  __device__ __forceinline__ bool filtered(const Pre& p) const { return p.m; }
   __device__ __forceinline__ void row(uint64_t i, DT sum, const Pre& p, double& a0, double& a1) const
   {
     DT v = dfma(sum, DT(1), DT(0));
@@ -243,6 +260,7 @@ struct EpiDefect
     bool m;
   };
   __device__ __forceinline__ Pre pre(uint64_t i) const { return Pre{rhs[i], first.load(i), is_masked(mask, i)}; }
+  __device__ __forceinline__ bool filtered(const Pre& p) const { return p.m; }
   __device__ __forceinline__ void row(uint64_t i, DT sum, const Pre& p, double& a0, double&) const
   {
     DT v = dfma(sum, DT(-1), p.rhs);
@@ -268,6 +286,7 @@ struct EpiProlAdd
     bool m;
   };
   __device__ __forceinline__ Pre pre(uint64_t i) const { return Pre{sol[i], is_masked(mask, i)}; }
+  __device__ __forceinline__ bool filtered(const Pre& p) const { return p.m; }
   __device__ __forceinline__ void row(uint64_t i, DT sum, const Pre& p, double&, double&) const
   {
     DT c = dfma(sum, DT(1), DT(0));
@@ -302,14 +321,12 @@ struct EpiSmooth
     DT rhs, inv, xk, acc, w;
     bool m;
   };
-  __device__ __forceinline__ Pre pre(uint64_t i) const
+  __device__ __forceinline__ Pre pre(uint64_t i) const { return pre(i, mode != 1 ? xk[i] : DT(0)); }
+  // the same where the caller holds xk[i]
+  __device__ __forceinline__ Pre pre(uint64_t i, DT xk_i) const
   {
-    Pre p{rhs[i], DT(0), DT(0), DT(0), DT(0), is_masked(mask, i)};
-    if(mode != 1)
-    {
-      p.inv = inv[i];
-      p.xk = xk[i];
-    }
+    Pre p{rhs[i], DT(0), xk_i, DT(0), DT(0), is_masked(mask, i)};
+    if(mode != 1) p.inv = inv[i];
     if(mode == 2)
     {
       p.acc = out[i];
@@ -317,6 +334,7 @@ struct EpiSmooth
     }
     return p;
   }
+  __device__ __forceinline__ bool filtered(const Pre& p) const { return p.m; }
   __device__ __forceinline__ void row(uint64_t i, DT sum, const Pre& p, double&, double& a1) const
   {
     DT d = dfma(sum, DT(-1), p.rhs);
@@ -555,6 +573,8 @@ __device__ __forceinline__ float wave_shift(float v)
 // x[row + c + 1] the right lane's: one load per triple and two wave shifts.
 constexpr int kMaxTrip = 10;
 constexpr uint32_t kDiagNone = 255u;   // slot without an entry
+// uniform-stencil march: from this many one-plane workgroups on, a lane takes three planes
+constexpr uint64_t kSten3 = 1024;
 
 // SpMV-type row loop over the diagonal plan: the slots run in ascending offset order (=
 // ascending columns, the CSR order), each lane adds its entry of a slot if it has one.
@@ -655,6 +675,178 @@ __global__ __launch_bounds__(kThreads) void k_sell_diag_rows(const DT* __restric
     }
   }
   grid_reduce_finish(gr, acc0, acc1);
+}
+
+// Uniform stencil rows (diagonal plans with grid_n1 set): every interior row of the n1^DIM grid
+// holds the same 3^DIM values, so it needs neither code words nor table lookups; a lane
+// marches over ZC consecutive planes (3D; lines in 2D) and loads x once per plane instead of
+// three times.  A wave covers kHaloRows consecutive positions of a plane (lanes 0 and 63: halo),
+// loads the 3 triple centres (3D; 1 in 2D) of ZC + 2 planes and all its rows' operands at once,
+// and gets the left / right values by wave shifts.  Each plane adds its taps to the rows of the
+// plane above (taps 0..8), its own (9..17) and the plane below (18..26): every sum runs in
+// ascending column order, bit-identical to the plan's rows.
+//
+// What bounds it: the Jacobi step of 3D Q1 level 7 was held up by its 9 triple loads and 7 code
+// words a row, 20 loads in flight a row for 32 bytes of vectors (30.9 us; FP32 20.3 us).
+// Marching 3 planes a lane loads 5 x values a row: 19 us (FP32 11.3), 3.6 TB/s of the vectors,
+// still latency at 5 waves a SIMD.  Two planes 22 us, four 20 us, eight 27 us (registers).
+// Where the grid has too few rows to fill the chip one plane a lane is best (3D level 5 3.3
+// against 3.7 us; level 6 the other way, 6.5 against 5.6 us): kSten3.  2D level 8 4.5 -> 2.9 us.
+//
+// Positions are flat in the plane, so the values at a plane's edges are of the wrong row; the
+// rows they belong to are boundary rows.  A boundary row that the epilogue filters does not
+// use its sum and is finished in place; the others are summed from their codes at the end, one
+// lane per boundary row.
+__host__ __device__ inline uint32_t grid_boundary_rows(int dim, uint32_t n1)
+{
+  return dim == 3 ? 2 * n1 * n1 + (n1 - 2) * (4 * n1 - 4) : 4 * n1 - 4;
+}
+
+// the b-th boundary node of an n1^DIM grid
+template<int DIM>
+__device__ __forceinline__ uint32_t grid_boundary_row(uint32_t b, uint32_t n1)
+{
+  auto ring = [n1](uint32_t k) -> uint32_t {   // the k-th boundary node of an n1 x n1 plane
+    if(k < n1) return k;
+    if(k < 2 * n1) return (n1 - 1) * n1 + (k - n1);
+    k -= 2 * n1;
+    return (1 + (k >> 1)) * n1 + ((k & 1) ? n1 - 1 : 0);
+  };
+  if(DIM == 2) return ring(b);
+  const uint32_t P = n1 * n1;
+  if(b < P) return b;
+  if(b < 2 * P) return (n1 - 1) * P + (b - P);
+  b -= 2 * P;
+  return (1 + b / (4 * n1 - 4)) * P + ring(b % (4 * n1 - 4));
+}
+
+// offset of the interior rows' values behind the pair table and the diagonal metadata
+template<typename DT>
+__host__ __device__ constexpr size_t sten_offset()
+{
+  return (256 * sizeof(DT) + (256 + 1 + kMaxTrip) * sizeof(int) + 7) & ~size_t(7);
+}
+
+template<typename DT, class Epi, int DIM, int ZC>
+__global__ __launch_bounds__(kThreads) void k_sten_rows(const DT* __restrict__ tab, const uint32_t* __restrict__ codes,
+                                                        int n1, const DT* __restrict__ x, uint32_t rows, Epi epi,
+                                                        GridReduce gr)
+{
+  constexpr int NT = DIM == 3 ? 9 : 3, NL = DIM == 3 ? 3 : 1, NW = (3 * NT + 3) / 4;
+  constexpr int kPre = ZC + 2;
+  const DT* __restrict__ sten = reinterpret_cast<const DT*>(reinterpret_cast<const char*>(tab) + sten_offset<DT>());
+  const int32_t m = n1, P = DIM == 3 ? m * m : m, last = int32_t(rows) - 1;
+  const uint32_t ngrp = (uint32_t(P) + kHaloChunk - 1) / kHaloChunk, nzc = (uint32_t(m) + ZC - 1) / ZC;
+  const uint32_t nmarch = ngrp * nzc, nbnd = grid_boundary_rows(DIM, uint32_t(m));
+  const XcdRange xr = xcd_range(nmarch);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double acc0 = 0.0, acc1 = 0.0;
+  epi.begin();
+  for(uint64_t item = xr.first; item < xr.end; item += xr.stride)
+  {
+    const uint32_t zc = uint32_t(item) / ngrp, g = uint32_t(item) - zc * ngrp;
+    const int32_t p = int32_t(g * kHaloChunk) + wave * kHaloRows + lane - 1, z0 = int32_t(zc) * ZC;
+    const bool mine = lane >= 1 && lane <= kHaloRows && p < P;
+    DT cen[kPre][NL];
+#pragma unroll
+    for(int j = 0; j < kPre; ++j)
+#pragma unroll
+      for(int d = 0; d < NL; ++d)
+      {
+        int32_t i = (z0 - 1 + j) * P + p + (DIM == 3 ? (d - 1) * m : 0);
+        i = i < 0 ? 0 : (i > last ? last : i);
+        // 32-bit byte offsets from the uniform base (at most 2^28 rows): one register an address
+        cen[j][d] = *reinterpret_cast<const DT*>(reinterpret_cast<const char*>(x) + uint32_t(i) * uint32_t(sizeof(DT)));
+      }
+    typename Epi::Pre pf[ZC];
+#pragma unroll
+    for(int j = 0; j < ZC; ++j)
+      if(mine && z0 + j < m)
+      {
+        const uint64_t row = uint64_t(uint32_t((z0 + j) * P + p));
+        if constexpr(EpiCentre<Epi, DT>::on)
+          pf[j] = epi.pre(row, cen[j + 1][NL / 2]);
+        else
+          pf[j] = epi.pre(row);
+      }
+    const int32_t px = DIM == 3 ? p % m : p, py = DIM == 3 ? p / m : 1;
+    const bool inner = px > 0 && px < m - 1 && (DIM == 2 || (py > 0 && py < m - 1));
+    DT acc[ZC];
+#pragma unroll
+    for(int j = 0; j < kPre; ++j)
+    {
+      DT v[NT];
+#pragma unroll
+      for(int d = 0; d < NL; ++d)
+      {
+        v[3 * d] = wave_shift<kDppWaveShr1>(cen[j][d]);
+        v[3 * d + 1] = cen[j][d];
+        v[3 * d + 2] = wave_shift<kDppWaveShl1>(cen[j][d]);
+      }
+      // plane z0 - 1 + j: the last taps of the row below it, the middle ones of its own, the
+      // first of the row above
+#pragma unroll
+      for(int u = 2; u >= 0; --u)
+        if(j - u >= 0 && j - u < ZC)
+        {
+          DT s = u == 0 ? DT(0) : acc[j - u];
+#pragma unroll
+          for(int t = 0; t < 3 * NL; ++t) s = dfma(sten[3 * NL * u + t], v[t], s);
+          acc[j - u] = s;
+        }
+      if(j >= 2)
+      {
+        const int32_t z = z0 + j - 2;
+        if(mine && z < m && ((inner && z > 0 && z < m - 1) || epi.filtered(pf[j - 2])))
+          epi.row(uint64_t(uint32_t(z * P + p)), acc[j - 2], pf[j - 2], acc0, acc1);
+      }
+    }
+  }
+  for(uint32_t b = blockIdx.x * kThreads + threadIdx.x; b < nbnd; b += gridDim.x * kThreads)
+  {
+    const uint32_t row = grid_boundary_row<DIM>(b, uint32_t(m));
+    const typename Epi::Pre pf = epi.pre(row);
+    if(epi.filtered(pf)) continue;   // finished in place
+    const uint32_t* cw = codes + uint64_t(row >> 6) * 64 * NW + (row & 63);
+    DT sum = DT(0);
+#pragma unroll
+    for(int t = 0; t < 3 * NT; ++t)
+    {
+      const uint32_t c = (cw[(t >> 2) * 64] >> (8 * (t & 3))) & 255u;
+      const int dx = t % 3 - 1, dy = DIM == 3 ? (t / 3) % 3 - 1 : t / 3 - 1, dz = DIM == 3 ? t / 9 - 1 : 0;
+      if(c != kDiagNone) sum = dfma(tab[c], x[int32_t(row) + dx + dy * m + dz * P], sum);
+    }
+    epi.row(row, sum, pf, acc0, acc1);
+  }
+  grid_reduce_finish(gr, acc0, acc1);
+}
+
+// the march of a uniform-stencil plan
+template<typename DT, class Epi, class M>
+int launch_sten(hipStream_t s, const M* A, const DT* x, const Epi& epi, const GridReduce& gr, const char* name)
+{
+  const uint32_t n1 = A->grid_n1, dim = A->grid_dim;
+  const uint32_t P = dim == 3 ? n1 * n1 : n1, ngrp = (P + kHaloChunk - 1) / kHaloChunk;
+  auto go = [&](auto zc, auto d) {
+    constexpr int ZC = decltype(zc)::value, DIM = decltype(d)::value;
+    const uint64_t items = uint64_t(ngrp) * ((n1 + ZC - 1) / ZC);
+    const int grid = int(items < uint64_t(kMaxGrid) ? items : uint64_t(kMaxGrid));
+    const GridReduce gd = reduce_for_grid(gr, uint64_t(grid));
+    hipLaunchKernelGGL((k_sten_rows<DT, Epi, DIM, ZC>), dim3(grid), dim3(kThreads), 0, s,
+                       reinterpret_cast<const DT*>(A->val), static_cast<const uint32_t*>(A->col), int(n1), x,
+                       uint32_t(A->rows), epi, gd);
+    finish_reduce(s, gd, uint64_t(grid));
+    return check_launch(name);
+  };
+  using std::integral_constant;
+  const uint64_t wg1 = uint64_t(ngrp) * n1;   // workgroups with one plane a lane
+  if(dim == 3)
+  {
+    if(wg1 >= kSten3) return go(integral_constant<int, 3>(), integral_constant<int, 3>());
+    return go(integral_constant<int, 1>(), integral_constant<int, 3>());
+  }
+  if(wg1 >= kSten3) return go(integral_constant<int, 3>(), integral_constant<int, 2>());
+  return go(integral_constant<int, 1>(), integral_constant<int, 2>());
 }
 
 // d-linear injection between structured grids (FEAT_FMT_DLINEAR): row sums formed from the
@@ -913,6 +1105,7 @@ int launch_mat(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gri
       finish_reduce(s, gd, uint64_t(grid));
       return check_launch(name);
     }
+    if(A->index == FEAT_IDX_DIAG && A->grid_n1) return launch_sten<DT>(s, A, x, epi, gr, name);
     if(A->index == FEAT_IDX_DIAG)
     {
       // chunks of kHaloChunk rows (62 per wave); a dot or norm is summed per chunk, so it
@@ -1200,6 +1393,25 @@ __global__ void k_sell_fill_code(const double* val, const uint64_t* col, const u
         codes[p] = 0;
         scol[p] = DELTA ? CT(0) : CT(r);
       }
+    }
+  }
+}
+
+// Uniform-stencil check of a diagonal plan's codes: 1 in *bad where an interior row of the n1^dim
+// grid differs from row `ref`, or a code of row `ref` is empty (set-up only)
+__global__ void k_sten_check(const uint32_t* codes, uint32_t nw, uint32_t nslot, int dim, uint32_t n1, uint64_t rows,
+                             uint64_t ref, int* bad)
+{
+  const uint32_t* rw = codes + (ref >> 6) * 64 * nw + (ref & 63);
+  for(uint64_t r = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; r < rows; r += uint64_t(gridDim.x) * blockDim.x)
+  {
+    const uint64_t fx = r % n1, fy = (r / n1) % n1, fz = dim == 3 ? r / (uint64_t(n1) * n1) : 1;
+    if(fx == 0 || fx == n1 - 1 || fy == 0 || fy == n1 - 1 || (dim == 3 && (fz == 0 || fz == n1 - 1))) continue;
+    const uint32_t* cw = codes + (r >> 6) * 64 * nw + (r & 63);
+    for(uint32_t t = 0; t < nslot; ++t)
+    {
+      const uint32_t c = (cw[(t >> 2) * 64] >> (8 * (t & 3))) & 255u, cr = (rw[(t >> 2) * 64] >> (8 * (t & 3))) & 255u;
+      if(c != cr || cr == kDiagNone) *bad = 1;
     }
   }
 }
@@ -2290,7 +2502,7 @@ int dict_create(feat_handle_t h, const feat_csr_f64_t* A, const std::vector<uint
   if(rc) { cleanup(); return rc; }
   // pair table: values in the plan's arithmetic type, then the offsets as int32, then
   // the diagonal plan's metadata (count, offsets, kinds)
-  std::vector<unsigned char> htab(256 * sizeof(DT) + (256 + 1 + kMaxTrip) * sizeof(int), 0);
+  std::vector<unsigned char> htab(sten_offset<DT>() + 27 * sizeof(DT), 0);
   DT* tv = reinterpret_cast<DT*>(htab.data());
   int* td = reinterpret_cast<int*>(htab.data() + 256 * sizeof(DT));
   uint32_t np = 0;
@@ -2380,12 +2592,50 @@ int dict_create(feat_handle_t h, const feat_csr_f64_t* A, const std::vector<uint
     cleanup();
     return dict_create<DT>(h, A, hmax, rlen, out, name, flags | FEAT_SELL_NO_DIAG);
   }
+  // uniform stencil: the offsets of the 3^dim neighbours on an n1^dim grid, and the same codes in
+  // every interior row; the values of those rows go behind the table
+  uint32_t grid_n1 = 0, grid_dim = 0;
+  if(!rc && diag && n == A->cols && n < (uint64_t(1) << 28))
+  {
+    for(uint32_t d = 3; d >= 2 && !grid_n1; --d)
+    {
+      const uint64_t q = uint64_t(std::llround(d == 3 ? std::cbrt(double(n)) : std::sqrt(double(n))));
+      if(q < 3 || (d == 3 ? q * q * q : q * q) != n || centres.size() != (d == 3 ? 9u : 3u)) continue;
+      bool same = true;
+      for(size_t g = 0; g < centres.size(); ++g)
+        same = same && centres[g] == (d == 3 ? (int(g / 3) - 1) * int(q * q) + (int(g % 3) - 1) * int(q) : (int(g) - 1) * int(q));
+      if(!same) continue;
+      const uint64_t ref = d == 3 ? q * q + q + 1 : q + 1;
+      uint32_t bad = 0;
+      rc = check_hip(hipMemsetAsync(state, 0, sizeof(uint32_t), h->stream), "memset");
+      if(rc) break;
+      hipLaunchKernelGGL(k_sten_check, dim3(grid_for(n)), dim3(kThreads), 0, h->stream, codes, dw, uint32_t(nslot),
+                         int(d), uint32_t(q), n, ref, (int*)state);
+      std::vector<uint32_t> words_of(dw);
+      rc = check_launch(name);
+      if(!rc) rc = check_hip(hipMemcpyAsync(&bad, state, sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream), "copy");
+      if(!rc)
+        rc = check_hip(hipMemcpy2DAsync(words_of.data(), sizeof(uint32_t), codes + (ref >> 6) * 64 * dw + (ref & 63),
+                                        64 * sizeof(uint32_t), sizeof(uint32_t), dw, hipMemcpyDeviceToHost, h->stream), "copy");
+      if(!rc) rc = check_hip(hipStreamSynchronize(h->stream), "sync");
+      if(rc || bad) break;
+      std::vector<DT> sv(nslot);
+      for(uint64_t t = 0; t < nslot; ++t) sv[t] = tv[(words_of[t >> 2] >> (8 * (t & 3))) & 255u];
+      rc = check_hip(hipMemcpyAsync(reinterpret_cast<char*>(table) + sten_offset<DT>(), sv.data(), sizeof(DT) * nslot,
+                                    hipMemcpyHostToDevice, h->stream), "copy");
+      if(!rc) rc = check_hip(hipStreamSynchronize(h->stream), "sync");
+      grid_n1 = uint32_t(q);
+      grid_dim = d;
+    }
+  }
   for(void** p : {(void**)&vtab, (void**)&dtab, (void**)&state, (void**)&present, (void**)&maps})
   {
     (void)hipFree(*p);
     *p = nullptr;
   }
   if(rc) { cleanup(); return rc; }
+  out->grid_n1 = grid_n1;
+  out->grid_dim = grid_dim;
   out->format = FEAT_FMT_SELL;
   out->index = diag ? FEAT_IDX_DIAG : FEAT_IDX_DICT;
   out->slice_words = diag ? dw : (uniform ? uint32_t(maxw) : 0u);

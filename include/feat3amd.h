@@ -279,6 +279,11 @@ typedef struct {
   uint32_t slice_words;      /* pair-dictionary plans: code words per lane in
                                 every slice (slice s at s * 64 * slice_words),
                                 0: per-slice offsets in ptr                   */
+  uint32_t grid_n1;          /* set by feat_sell_create_*, 0 otherwise.  FEAT_IDX_DIAG:
+                                the rows are the clipped 3^grid_dim-point stencils of a
+                                grid with grid_n1 nodes per side, the same values in
+                                every interior row                            */
+  uint32_t grid_dim;
 } feat_matrix_f64_t;
 
 typedef struct {             /* FP32 arithmetic (mixed-precision inner solver) */
@@ -292,6 +297,7 @@ typedef struct {             /* FP32 arithmetic (mixed-precision inner solver) *
   float scale;               /* row sums are multiplied by this power of two  */
   int tune;                  /* SELL launch shape, 0 = default                */
   uint32_t slice_words;      /* as feat_matrix_f64_t::slice_words             */
+  uint32_t grid_n1, grid_dim;   /* as feat_matrix_f64_t                       */
 } feat_matrix_f32_t;
 
 /* A CSR descriptor (no copy) of the caller's arrays. */
