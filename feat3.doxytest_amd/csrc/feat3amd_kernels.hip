@@ -941,7 +941,16 @@ __global__ __launch_bounds__(kThreads) void k_dlinear_rows(int dim, int n1, cons
 // which is the CSR order the plan was checked against at set-up.  The value arrays are
 // streamed once (nontemporal loads); x stays in L2.  Indices and byte offsets are 32-bit:
 // the plan requires 27 * rows * 8 B < 4 GiB (fewer than 19.8 M rows).
-template<typename DT, typename VT, class Epi, int DIM>
+//
+// SYM (the plan's values are symmetric bit for bit, checked at set-up): the entry of row i at a
+// negative offset is the entry of row i + offset at the opposite slot, so only the slots from
+// the diagonal on are streamed, 14 of 27, and the others are read where the rows below have just
+// brought them into the XCD's L2 (consecutive chunks run on one XCD).  The value arrays go
+// through the caches then.  A smoother call of 4 steps on 129^3 nodes: FP64 461 -> 337 us
+// (3.7 TB/s of the bytes left), FP32 215 -> 115 us (5.4 TB/s), FP16 values 150 -> 100 us; on
+// 65^3 nodes 72 -> 52, 34 -> 28, 31 -> 27 us.  Marching over planes as k_sten_rows does (3 loads
+// of x a row instead of 27) gained nothing here and cost 20 to 50 % on 65^3 nodes.
+template<typename DT, typename VT, class Epi, int DIM, bool SYM>
 __global__ __launch_bounds__(kThreads) void k_band_rows(const VT* __restrict__ val, int n1,
                                                         const DT* __restrict__ x, uint64_t rows, DT scale,
                                                         Epi epi, GridReduce gr)
@@ -979,16 +988,26 @@ __global__ __launch_bounds__(kThreads) void k_band_rows(const VT* __restrict__ v
                       (dz < 0 ? lz : dz > 0 ? hz : true);
       // 32-bit byte offsets from one base per array (the plan keeps its values below 4 GiB):
       // one offset register per load instead of a 64-bit address
-      const VT* vp = (const VT*)((const char*)val + (ro + uint32_t(t) * st));
+      const int32_t nb = i + dx + dy * m + dz * mm;
+      const bool mirror = SYM && t < NS / 2;
+      const VT* vp = (const VT*)((const char*)val + (mirror ? uint32_t(sizeof(VT) == 2 && !on ? i : nb) * uint32_t(sizeof(VT)) +
+                                                                  uint32_t(NS - 1 - t) * st
+                                                            : ro + uint32_t(t) * st));
+      auto load = [&]() -> VT {
+        if constexpr(SYM)
+          return *vp;
+        else
+          return __builtin_nontemporal_load(vp);
+      };
       if constexpr(sizeof(VT) == 2)
       {
-        v[t] = __builtin_nontemporal_load(vp);
-        xv[t] = *(const DT*)((const char*)x + uint32_t(on ? i + dx + dy * m + dz * mm : i) * uint32_t(sizeof(DT)));
+        v[t] = load();
+        xv[t] = *(const DT*)((const char*)x + uint32_t(on ? nb : i) * uint32_t(sizeof(DT)));
       }
       else
       {
-        v[t] = on ? __builtin_nontemporal_load(vp) : VT(0);
-        xv[t] = on ? *(const DT*)((const char*)x + uint32_t(i + dx + dy * m + dz * mm) * uint32_t(sizeof(DT))) : DT(0);
+        v[t] = on ? load() : VT(0);
+        xv[t] = on ? *(const DT*)((const char*)x + uint32_t(nb) * uint32_t(sizeof(DT))) : DT(0);
       }
     }
     DT sum = DT(0);
@@ -1047,23 +1066,32 @@ int launch_mat(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gri
     const int n1 = int(A->slice_words);
     const bool d3 = band_dim(A->rows, A->slice_words) == 3;
     const DT sc = DT(A->scale);
+    auto go = [&](auto v, auto dim, auto sym) {
+      hipLaunchKernelGGL((k_band_rows<DT, std::remove_const_t<std::remove_pointer_t<decltype(v)>>, Epi, decltype(dim)::value,
+                                      decltype(sym)::value>),
+                         dim3(grid), dim3(kThreads), 0, s, v, n1, x, A->rows, sc, epi, gd);
+    };
+    auto by_shape = [&](auto v) {
+      using std::integral_constant;
+      const bool sym = A->grid_n1 != 0;
+      if(d3 && sym)
+        go(v, integral_constant<int, 3>(), std::true_type());
+      else if(d3)
+        go(v, integral_constant<int, 3>(), std::false_type());
+      else if(sym)
+        go(v, integral_constant<int, 2>(), std::true_type());
+      else
+        go(v, integral_constant<int, 2>(), std::false_type());
+    };
     if(A->value_kind == FEAT_VAL_F16)
     {
       if constexpr(!std::is_same<DT, float>::value)
         return fail(FEAT_ERR_UNSUPPORTED, "FP16 values need FP32 arithmetic");
       else
-      {
-        const uint16_t* vh = (const uint16_t*)(const void*)A->val;
-        if(d3)
-          hipLaunchKernelGGL((k_band_rows<DT, uint16_t, Epi, 3>), dim3(grid), dim3(kThreads), 0, s, vh, n1, x, A->rows, sc, epi, gd);
-        else
-          hipLaunchKernelGGL((k_band_rows<DT, uint16_t, Epi, 2>), dim3(grid), dim3(kThreads), 0, s, vh, n1, x, A->rows, sc, epi, gd);
-      }
+        by_shape((const uint16_t*)(const void*)A->val);
     }
-    else if(d3)
-      hipLaunchKernelGGL((k_band_rows<DT, DT, Epi, 3>), dim3(grid), dim3(kThreads), 0, s, A->val, n1, x, A->rows, sc, epi, gd);
     else
-      hipLaunchKernelGGL((k_band_rows<DT, DT, Epi, 2>), dim3(grid), dim3(kThreads), 0, s, A->val, n1, x, A->rows, sc, epi, gd);
+      by_shape(A->val);
     finish_reduce(s, gd, uint64_t(grid));
     return check_launch(name);
   }
@@ -1353,6 +1381,28 @@ __host__ __device__ inline DT key_value(uint64_t k)
     return __builtin_bit_cast(DT, uint32_t(k));
   else
     return __builtin_bit_cast(DT, uint16_t(k));
+}
+
+// Symmetry of a banded plan's values: 1 in *bad where an entry differs in its bits from the
+// entry of the neighbour's row at the opposite slot (set-up only)
+template<typename DT>
+__global__ void k_band_symmetric(const DT* bval, uint64_t rows, int dim, int64_t n1, int* bad)
+{
+  const int ns = dim == 3 ? 27 : 9;
+  for(uint64_t r = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; r < rows; r += uint64_t(gridDim.x) * blockDim.x)
+  {
+    const int64_t i = int64_t(r);
+    const int64_t fx = i % n1, fy = (i / n1) % n1, fz = dim == 3 ? i / (n1 * n1) : 0;
+    bool ok = true;
+    for(int t = 0; t < ns / 2; ++t)
+    {
+      const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = dim == 3 ? t / 9 - 1 : 0;
+      if(fx + dx < 0 || fx + dx >= n1 || fy + dy < 0 || fy + dy >= n1 || fz + dz < 0 || fz + dz >= n1) continue;
+      const int64_t nb = i + dx + dy * n1 + dz * n1 * n1;
+      ok = ok && value_key<DT>(bval[uint64_t(t) * rows + r]) == value_key<DT>(bval[uint64_t(ns - 1 - t) * rows + uint64_t(nb)]);
+    }
+    if(!ok) *bad = 1;
+  }
 }
 
 // Value-code fill: the SELL layout of k_sell_fill with each value replaced by its index
@@ -2699,10 +2749,13 @@ int band_create(feat_handle_t h, const feat_csr_f64_t* A, float scale, float inv
       n1 = cand[c][1];
     }
   }
-  if(bad) (void)hipFree(bad);
-  if(rc) return rc;
-  if(!dim) return FEAT_ERR_UNSUPPORTED;
+  if(rc || !dim)
+  {
+    if(bad) (void)hipFree(bad);
+    return rc ? rc : FEAT_ERR_UNSUPPORTED;
+  }
   const uint64_t ns = dim == 3 ? 27 : 9;
+  int asym = 1;
   DT* bval = nullptr;
   rc = check_hip(hipMalloc(&bval, sizeof(DT) * ns * n), "banded plan values");
   if(!rc)
@@ -2711,7 +2764,15 @@ int band_create(feat_handle_t h, const feat_csr_f64_t* A, float scale, float inv
                        int64_t(n1), bval, inv_scale);
     rc = check_launch("banded plan fill");
   }
+  if(!rc) rc = check_hip(hipMemsetAsync(bad, 0, sizeof(int), h->stream), "memset");
+  if(!rc)
+  {
+    hipLaunchKernelGGL((k_band_symmetric<DT>), dim3(grid_for(n)), dim3(kThreads), 0, h->stream, bval, n, dim, int64_t(n1), bad);
+    rc = check_launch("banded plan symmetry");
+  }
+  if(!rc) rc = check_hip(hipMemcpyAsync(&asym, bad, sizeof(int), hipMemcpyDeviceToHost, h->stream), "copy");
   if(!rc) rc = check_hip(hipStreamSynchronize(h->stream), "sync");
+  (void)hipFree(bad);
   if(rc)
   {
     if(bval) (void)hipFree(bval);
@@ -2730,6 +2791,8 @@ int band_create(feat_handle_t h, const feat_csr_f64_t* A, float scale, float inv
   out->scale = scale;
   out->tune = 0;
   out->slice_words = uint32_t(n1);
+  out->grid_n1 = asym ? 0u : uint32_t(n1);
+  out->grid_dim = asym ? 0u : uint32_t(dim);
   return FEAT_OK;
 }
 

@@ -282,7 +282,8 @@ typedef struct {
   uint32_t grid_n1;          /* set by feat_sell_create_*, 0 otherwise.  FEAT_IDX_DIAG:
                                 the rows are the clipped 3^grid_dim-point stencils of a
                                 grid with grid_n1 nodes per side, the same values in
-                                every interior row                            */
+                                every interior row.  FEAT_FMT_BANDED: the values are
+                                symmetric bit for bit                         */
   uint32_t grid_dim;
 } feat_matrix_f64_t;
 
