@@ -8,6 +8,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <type_traits>
 
@@ -264,6 +265,9 @@ struct feat_handle_s
   uint32_t* counter;
   double* scal;       // scratch device scalars
   double* host;       // pinned host scalars
+  // stream-ordered buffers of the transposed apply (made at its first call, bounded)
+  std::mutex pool_mutex;
+  hipMemPool_t pool = nullptr;
 };
 
 namespace {

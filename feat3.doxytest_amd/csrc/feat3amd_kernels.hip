@@ -1948,6 +1948,7 @@ int feat_handle_destroy(feat_handle_t h)
   if(h->scal) (void)hipFree(h->scal);
   if(h->host) (void)hipHostFree(h->host);
   if(h->event) (void)hipEventDestroy(h->event);
+  if(h->pool) (void)hipMemPoolDestroy(h->pool);
   if(h->own_stream && h->stream) (void)hipStreamDestroy(h->stream);
   delete h;
   return FEAT_OK;

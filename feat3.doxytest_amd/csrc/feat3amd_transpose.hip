@@ -3,22 +3,29 @@
 // The reference's generic transposed apply (arch/apply_generic.hpp:37-53) is
 //     r = (b/a) * (|b| < eps ? 0 : y);   r[col[i]] += val[i] * x[row];   r = a * r
 // with the scatter running over the rows in order, so every r[c] accumulates its
-// column's entries in ascending entry order.  Here each call builds the column
-// order of the entries (a stable radix sort of the column indices, so entries of
-// one column keep their CSR order) and then one lane per column gathers its
-// entries in that order: the same additions in the same order, with no atomics,
-// so the result is deterministic and bit-identical to the sequential loop.
-// The call allocates its sort buffers stream-ordered (this path is set-up work in
-// the reference's solvers, which form R = P^T explicitly); the allocation-free variant
-// keeps them in a static device array instead.
+// column's entries in ascending entry order.  Here each call collects the entries of every
+// column (entries counted per column, the counts summed up, entry and row number written to
+// the column's place), sorts each column's short list by entry number and adds it up in that
+// order: the same additions in the same order, with no atomics on values, so the result is
+// deterministic and bit-identical to the sequential loop.
+//
+// A stable radix sort of all entries by column, with one lane per column following the sorted
+// entries one dependent load at a time, took 0.68 ms on 7.1 M entries (3D Q1 level 6), 0.35 ms
+// of it the gather; the lists cost one pass of counting atomics (119 us, the largest part now)
+// and one of placing (67 us) instead of three sort passes, and a workgroup loads all entries of
+// its 32 columns at once (63 us): 0.32 ms in all.
+//
+// The buffers of the allocating form come stream-ordered from a pool of the handle's own, which
+// keeps up to kTrPoolBytes between calls (the device's default pool gives everything back at
+// every synchronisation: 2.3 ms for a call that is waited for, 0.42 ms now); the
+// allocation-free variant keeps them in a static device array instead.
 #include "feat3amd_common.hpp"
 
+#include <algorithm>
 #include <mutex>
 
-#include <hipcub/hipcub.hpp>
-
 // Scratch of the allocation-free variant (feat_csr_apply_transposed_noalloc_f64_u64): the
-// sort buffers live in this file-scope device array, one copy per GPU, held until the
+// column lists live in this file-scope device array, one copy per GPU, held until the
 // process ends.  Host code never passes `scratch` itself to a kernel or copy (on the host
 // the name is only a stand-in for the symbol): it uses the per-device address that
 // hipGetSymbolAddress returned at handle creation.  Every call on one GPU shares that
@@ -28,6 +35,7 @@ static __device__ __align__(256) unsigned char scratch[FEAT_TR_NOALLOC_SCRATCH_B
 namespace {
 
 constexpr size_t kTrScratchBytes = size_t(FEAT_TR_NOALLOC_SCRATCH_BYTES);
+constexpr uint64_t kTrPoolBytes = uint64_t(256) << 20;   // most a handle keeps between calls
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mutex;
 void* g_scratch_ptr[kMaxDevices] = {};
@@ -39,57 +47,304 @@ void* scratch_of(int device)
   return g_scratch_ptr[device];
 }
 
-template<typename IT>
-__global__ void k_tr_keys(const IT* col, uint64_t nnz, uint32_t* keys, uint32_t* idx)
+constexpr uint32_t kTrScan = 1024;     // counts a workgroup scans
+constexpr uint32_t kTrTile = 4096;     // entries a workgroup places
+constexpr uint32_t kTrCols = 32;       // columns a workgroup adds up
+constexpr uint32_t kTrPer = kThreads / kTrCols;   // threads a column
+constexpr uint32_t kTrCap = 1024;      // entries it holds in LDS at a time (27-point rows: 864)
+constexpr uint32_t kTrShort = 64;      // longest list that is ordered by counting
+
+__global__ void k_tr_zero(uint32_t* p, uint64_t n)
 {
-  for(uint64_t e = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; e < nnz; e += uint64_t(gridDim.x) * blockDim.x)
+  for(uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x) p[i] = 0;
+}
+
+// cnt[c]: entries of column c; rank[e]: a number of its own for entry e within its column
+template<typename IT>
+__global__ __launch_bounds__(kThreads) void k_tr_count(const IT* __restrict__ col, uint64_t nnz, uint32_t* cnt,
+                                                       uint32_t* __restrict__ rank)
+{
+  const uint64_t stride = uint64_t(gridDim.x) * kThreads;
+  for(uint64_t e0 = blockIdx.x * uint64_t(kThreads) + threadIdx.x; e0 < nnz; e0 += 4 * stride)
   {
-    keys[e] = uint32_t(col[e]);
-    idx[e] = uint32_t(e);
+    IT c[4];
+    uint32_t k[4];
+#pragma unroll
+    for(int u = 0; u < 4; ++u) c[u] = e0 + u * stride < nnz ? col[e0 + u * stride] : IT(0);
+#pragma unroll
+    for(int u = 0; u < 4; ++u) k[u] = e0 + u * stride < nnz ? atomicAdd(cnt + c[u], 1u) : 0u;
+#pragma unroll
+    for(int u = 0; u < 4; ++u)
+      if(e0 + u * stride < nnz) rank[e0 + u * stride] = k[u];
   }
 }
 
-template<typename IT>
-__global__ void k_tr_row_of(const IT* rowptr, uint64_t rows, uint32_t* row_of)
+// exclusive sum over the workgroup's kThreads values
+__device__ uint32_t block_scan(uint32_t v, uint32_t* sh /* kThreads / 64 */, uint32_t& total)
 {
-  for(uint64_t r = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; r < rows; r += uint64_t(gridDim.x) * blockDim.x)
-    for(uint64_t e = uint64_t(rowptr[r]); e < uint64_t(rowptr[r + 1]); ++e) row_of[e] = uint32_t(r);
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  uint32_t s = v;
+  for(int d = 1; d < 64; d <<= 1)
+  {
+    const uint32_t t = __shfl_up(s, d, 64);
+    if(lane >= d) s += t;
+  }
+  if(lane == 63) sh[w] = s;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+  for(int i = 0; i < kThreads / 64; ++i)
+  {
+    if(i < w) before += sh[i];
+    total += sh[i];
+  }
+  __syncthreads();
+  return before + s - v;
 }
 
-// colptr[c] = first position of column c in the sorted keys (empty columns included)
-__global__ void k_tr_colptr(const uint32_t* keys, uint64_t nnz, uint64_t cols, uint32_t* colptr)
+__global__ __launch_bounds__(kThreads) void k_tr_sums(const uint32_t* cnt, uint64_t n, uint32_t* sums)
 {
-  for(uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i <= nnz; i += uint64_t(gridDim.x) * blockDim.x)
+  __shared__ uint32_t sh[kThreads / 64];
+  uint32_t v = 0, total;
+  for(uint32_t u = 0; u < kTrScan / kThreads; ++u)
   {
-    const int64_t kp = i == 0 ? -1 : int64_t(keys[i - 1]);
-    const int64_t kc = i == nnz ? int64_t(cols) : int64_t(keys[i]);
-    for(int64_t c = kp + 1; c <= kc; ++c) colptr[c] = uint32_t(i);
+    const uint64_t i = uint64_t(blockIdx.x) * kTrScan + u * kThreads + threadIdx.x;
+    if(i < n) v += cnt[i];
+  }
+  (void)block_scan(v, sh, total);
+  if(threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// exclusive sums of the nb workgroup sums, in place (one workgroup)
+__global__ __launch_bounds__(kThreads) void k_tr_scan_sums(uint32_t* sums, uint32_t nb)
+{
+  __shared__ uint32_t sh[kThreads / 64];
+  uint32_t carry = 0;
+  for(uint32_t i0 = 0; i0 < nb; i0 += kThreads)
+  {
+    const uint32_t i = i0 + threadIdx.x;
+    uint32_t total;
+    const uint32_t s = block_scan(i < nb ? sums[i] : 0u, sh, total);
+    if(i < nb) sums[i] = carry + s;
+    carry += total;
   }
 }
 
-template<typename DT>
-__global__ void k_tr_gather(DT* r, DT a, DT ba, const DT* x, const DT* y, int bzero, const DT* val,
-                            const uint32_t* colptr, const uint32_t* order, const uint32_t* row_of, uint64_t cols)
+// counts -> first positions, in place; ptr[n] = all entries
+__global__ __launch_bounds__(kThreads) void k_tr_colptr(uint32_t* ptr, uint64_t n, const uint32_t* sums, uint32_t nnz)
 {
-  for(uint64_t c = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; c < cols; c += uint64_t(gridDim.x) * blockDim.x)
+  __shared__ uint32_t sh[kThreads / 64];
+  uint32_t carry = sums[blockIdx.x];
+  for(uint32_t u = 0; u < kTrScan / kThreads; ++u)
   {
-    DT acc = ba * (bzero ? DT(0) : y[c]);
-    for(uint32_t k = colptr[c]; k < colptr[c + 1]; ++k)
+    const uint64_t i = uint64_t(blockIdx.x) * kTrScan + u * kThreads + threadIdx.x;
+    uint32_t total;
+    const uint32_t s = block_scan(i < n ? ptr[i] : 0u, sh, total);
+    if(i < n) ptr[i] = carry + s;
+    carry += total;
+  }
+  if(blockIdx.x == 0 && threadIdx.x == 0) ptr[n] = nnz;
+}
+
+// list[position] = entry number (high half) and row (low half): ascending words = ascending entries
+template<typename IT>
+__global__ __launch_bounds__(kThreads) void k_tr_place(const IT* __restrict__ col, const IT* __restrict__ rowptr,
+                                                       uint64_t rows, uint64_t nnz, const uint32_t* __restrict__ colptr,
+                                                       const uint32_t* __restrict__ rank, uint64_t* __restrict__ list)
+{
+  __shared__ uint32_t srp[kTrTile + 2];
+  __shared__ uint64_t sr[2];
+  for(uint64_t e0 = uint64_t(blockIdx.x) * kTrTile; e0 < nnz; e0 += uint64_t(gridDim.x) * kTrTile)
+  {
+    const uint64_t e1 = e0 + kTrTile < nnz ? e0 + kTrTile : nnz;
+    // the rows of the tile's first and last entry: the last r with rowptr[r] <= e
+    if(threadIdx.x < 2)
     {
-      const uint32_t e = order[k];
-      acc = dfma(val[e], x[row_of[e]], acc);
+      const uint64_t e = threadIdx.x ? e1 - 1 : e0;
+      uint64_t lo = 0, hi = rows;
+      while(hi - lo > 1)
+      {
+        const uint64_t mid = (lo + hi) >> 1;
+        if(uint64_t(rowptr[mid]) <= e)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      sr[threadIdx.x] = lo;
     }
-    r[c] = a * acc;
+    __syncthreads();
+    const uint64_t r0 = sr[0], nr = sr[1] - sr[0] + 1;
+    const bool in_lds = nr <= kTrTile + 1;
+    if(in_lds)
+      for(uint64_t i = threadIdx.x; i < nr; i += kThreads) srp[i] = uint32_t(rowptr[r0 + i]);
+    __syncthreads();
+    for(uint64_t e = e0 + threadIdx.x; e < e1; e += kThreads)
+    {
+      const uint64_t c = uint64_t(col[e]);
+      const uint32_t k = rank[e];
+      uint64_t lo = 0, hi = nr;
+      while(hi - lo > 1)
+      {
+        const uint64_t mid = (lo + hi) >> 1;
+        const uint64_t v = in_lds ? uint64_t(srp[mid]) : uint64_t(rowptr[r0 + mid]);
+        if(v <= e)
+          lo = mid;
+        else
+          hi = mid;
+      }
+      list[colptr[c] + k] = (e << 32) | (r0 + lo);
+    }
+    __syncthreads();
   }
 }
 
-template<typename T>
-int dev_alloc(T** p, uint64_t n, hipStream_t s)
+// ascending sort of a[0 .. n) by the whole workgroup (bitonic network; pairs with one end at or
+// beyond n are already in order, as if the missing words were larger than all)
+__device__ void block_sort(uint64_t* a, uint32_t n)
 {
-  return check_hip(hipMallocAsync(reinterpret_cast<void**>(p), sizeof(T) * (n ? n : 1), s), "transposed apply: buffer");
+  uint32_t p = 2;
+  for(; p < 2 * n && p; p <<= 1)
+  {
+    // first step of a merge: mirrored pairs, the further ones at distance d
+    for(uint32_t i = threadIdx.x; i < (n + p - 1) / p * (p / 2); i += kThreads)
+    {
+      const uint32_t b = i / (p / 2) * p, o = i % (p / 2), l = b + o, h = b + p - 1 - o;
+      if(h < n)
+      {
+        const uint64_t x = a[l], y = a[h];
+        if(y < x)
+        {
+          a[l] = y;
+          a[h] = x;
+        }
+      }
+    }
+    __syncthreads();
+    for(uint32_t d = p / 4; d; d >>= 1)
+    {
+      for(uint32_t i = threadIdx.x; i < (n + 2 * d - 1) / (2 * d) * d; i += kThreads)
+      {
+        const uint32_t l = i / d * 2 * d + i % d, h = l + d;
+        if(h < n)
+        {
+          const uint64_t x = a[l], y = a[h];
+          if(y < x)
+          {
+            a[l] = y;
+            a[h] = x;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
 }
 
-// 256-byte aligned bump layout inside the scratch array
+// kTrCols columns a workgroup, kTrPer threads a column.  A thread holds up to 4 entries of its
+// column's list at a time and counts the smaller entry numbers in it, while the entries' values
+// and x are on their way; both go to their place in LDS, and one lane a column adds them in
+// order.  (One lane a column sorting its list in LDS took 233 us instead of 63.)  Lists
+// longer than kTrShort are sorted by the workgroup, in place where they do not fit in LDS.
+template<typename DT>
+__global__ __launch_bounds__(kThreads) void k_tr_gather(DT* r, DT a, DT ba, const DT* x, const DT* y, int bzero,
+                                                        const DT* val, const uint32_t* colptr, uint64_t* list, uint64_t cols)
+{
+  __shared__ uint64_t sl[kTrCap];
+  __shared__ DT sv[kTrCap], sx[kTrCap];
+  __shared__ uint32_t cp[kTrCols + 1];
+  uint32_t* se = reinterpret_cast<uint32_t*>(sl);
+  const uint32_t t = threadIdx.x, tc = t / kTrPer, sub = t % kTrPer;
+  for(uint64_t c0 = uint64_t(blockIdx.x) * kTrCols; c0 < cols; c0 += uint64_t(gridDim.x) * kTrCols)
+  {
+    const uint32_t nc = cols - c0 < kTrCols ? uint32_t(cols - c0) : kTrCols;
+    if(t <= nc) cp[t] = colptr[c0 + t];
+    __syncthreads();
+    for(uint32_t c = 0; c < nc;)
+    {
+      // the next columns that fit together, or one long column
+      const uint32_t p0 = cp[c];
+      const bool lng = cp[c + 1] - p0 > kTrShort;
+      uint32_t ce = c + 1;
+      if(!lng)
+        while(ce < nc && cp[ce + 1] - p0 <= kTrCap && cp[ce + 1] - cp[ce] <= kTrShort) ++ce;
+      const uint32_t n = cp[ce] - p0;
+      DT acc = DT(0);
+      if(t < ce - c) acc = ba * (bzero ? DT(0) : y[c0 + c + t]);
+      if(!lng)
+      {
+        const bool on = tc < ce - c;
+        const uint32_t b = on ? cp[c + tc] - p0 : 0, e = on ? cp[c + tc + 1] - p0 : 0;
+        for(uint32_t i = b + sub; i < e; i += kTrPer) se[i] = uint32_t(list[p0 + i] >> 32);
+        __syncthreads();
+        for(uint32_t i0 = b + sub; i0 < e; i0 += 4 * kTrPer)
+        {
+          uint32_t en[4], rank[4];
+          DT v[4], xv[4];
+#pragma unroll
+          for(uint32_t u = 0; u < 4; ++u)
+          {
+            const uint32_t i = i0 + u * kTrPer;
+            const uint64_t w = i < e ? list[p0 + i] : list[p0 + i0];
+            en[u] = uint32_t(w >> 32);
+            v[u] = val[w >> 32];
+            xv[u] = x[uint32_t(w)];
+            rank[u] = 0;
+          }
+#pragma unroll 4
+          for(uint32_t j = b; j < e; ++j)
+          {
+            const uint32_t o = se[j];
+#pragma unroll
+            for(uint32_t u = 0; u < 4; ++u) rank[u] += o < en[u] ? 1u : 0u;
+          }
+#pragma unroll
+          for(uint32_t u = 0; u < 4; ++u)
+            if(i0 + u * kTrPer < e)
+            {
+              sv[b + rank[u]] = v[u];
+              sx[b + rank[u]] = xv[u];
+            }
+        }
+        __syncthreads();
+        if(t < ce - c)
+        {
+          const uint32_t bt = cp[c + t] - p0, et = cp[c + t + 1] - p0;
+#pragma unroll 4
+          for(uint32_t i = bt; i < et; ++i) acc = dfma(sv[i], sx[i], acc);
+        }
+      }
+      else
+      {
+        if(n > kTrCap) block_sort(list + p0, n);   // sorted where it lies
+        for(uint32_t q = 0; q < n; q += kTrCap)
+        {
+          const uint32_t m = n - q < kTrCap ? n - q : kTrCap;
+          for(uint32_t i = t; i < m; i += kThreads) sl[i] = list[p0 + q + i];
+          __syncthreads();
+          if(n <= kTrCap) block_sort(sl, n);
+          for(uint32_t i = t; i < m; i += kThreads)
+          {
+            const uint64_t w = sl[i];
+            sv[i] = val[w >> 32];
+            sx[i] = x[uint32_t(w)];
+          }
+          __syncthreads();
+          if(t == 0)
+          {
+#pragma unroll 4
+            for(uint32_t i = 0; i < m; ++i) acc = dfma(sv[i], sx[i], acc);
+          }
+          __syncthreads();
+        }
+      }
+      if(t < ce - c) r[c0 + c + t] = a * acc;
+      c = ce;
+      __syncthreads();
+    }
+  }
+}
+
+// 256-byte aligned bump layout inside one buffer
 struct ScratchLayout
 {
   size_t off = 0;
@@ -101,6 +356,47 @@ struct ScratchLayout
     return o;
   }
 };
+
+struct TrLayout
+{
+  size_t colptr, sums, rank, list, bytes;
+  uint32_t nb;
+  TrLayout(uint64_t cols, uint64_t nnz) : nb(uint32_t((cols + kTrScan - 1) / kTrScan))
+  {
+    ScratchLayout lay;
+    colptr = lay.take<uint32_t>(cols + 1);
+    sums = lay.take<uint32_t>(nb);
+    rank = lay.take<uint32_t>(nnz);
+    list = lay.take<uint64_t>(nnz);
+    bytes = lay.off;
+  }
+};
+
+// the transposed apply with its buffers at base (cols > 0)
+template<typename DT, typename IT>
+int tr_apply(hipStream_t s, unsigned char* base, const TrLayout& L, DT* r, DT a, const DT* x, DT b, bool bzero, const DT* y,
+             const DT* val, const IT* col, const IT* rowptr, uint64_t rows, uint64_t cols, uint64_t nnz, const char* name)
+{
+  uint32_t* colptr = reinterpret_cast<uint32_t*>(base + L.colptr);
+  uint32_t* sums = reinterpret_cast<uint32_t*>(base + L.sums);
+  uint32_t* rank = reinterpret_cast<uint32_t*>(base + L.rank);
+  uint64_t* list = reinterpret_cast<uint64_t*>(base + L.list);
+  hipLaunchKernelGGL(k_tr_zero, dim3(grid_for(cols + 1)), dim3(kThreads), 0, s, colptr, cols + 1);
+  if(nnz)
+  {
+    hipLaunchKernelGGL((k_tr_count<IT>), dim3(grid_for(nnz, 4)), dim3(kThreads), 0, s, col, nnz, colptr, rank);
+    hipLaunchKernelGGL(k_tr_sums, dim3(L.nb), dim3(kThreads), 0, s, colptr, cols, sums);
+    hipLaunchKernelGGL(k_tr_scan_sums, dim3(1), dim3(kThreads), 0, s, sums, L.nb);
+    hipLaunchKernelGGL(k_tr_colptr, dim3(L.nb), dim3(kThreads), 0, s, colptr, cols, sums, uint32_t(nnz));
+    const uint64_t tiles = (nnz + kTrTile - 1) / kTrTile;
+    hipLaunchKernelGGL((k_tr_place<IT>), dim3(unsigned(std::min<uint64_t>(tiles, kMaxGrid))), dim3(kThreads), 0, s, col,
+                       rowptr, rows, nnz, colptr, rank, list);
+  }
+  const uint64_t groups = (cols + kTrCols - 1) / kTrCols;
+  hipLaunchKernelGGL((k_tr_gather<DT>), dim3(unsigned(std::min<uint64_t>(groups, kMaxGrid))), dim3(kThreads), 0, s, r, a,
+                     DT(b / a), x, y, int(bzero), val, colptr, list, cols);
+  return check_launch(name);
+}
 
 } // namespace
 
@@ -130,49 +426,46 @@ int csr_apply_transposed_noalloc(feat_handle_t h, DT* r, DT a, const DT* x, DT b
   unsigned char* base = static_cast<unsigned char*>(scratch_of(h->device));
   if(!base) return fail(FEAT_ERR_NO_DEVICE, "csr_apply_transposed_noalloc: scratch not attached on the handle's device");
   if(!cols) return FEAT_OK;
-  hipStream_t s = h->stream;
-  int end_bit = 1;
-  while(end_bit < 32 && (uint64_t(1) << end_bit) < cols) ++end_bit;
-  ScratchLayout lay;
-  const size_t o_colptr = lay.take<uint32_t>(cols + 1);
-  const size_t o_k0 = lay.take<uint32_t>(nnz), o_k1 = lay.take<uint32_t>(nnz);
-  const size_t o_v0 = lay.take<uint32_t>(nnz), o_v1 = lay.take<uint32_t>(nnz);
-  const size_t o_row = lay.take<uint32_t>(nnz);
-  auto at = [&](size_t o) { return reinterpret_cast<uint32_t*>(base + o); };
-  hipcub::DoubleBuffer<uint32_t> dk(at(o_k0), at(o_k1)), dv(at(o_v0), at(o_v1));
-  size_t tmp_bytes = 0;
-  if(nnz)
-  {
-    const int rc = check_hip(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, dk, dv, int(nnz), 0, end_bit, s),
-                             "transposed apply: sort size");
-    if(rc) return rc;
-  }
-  const size_t o_tmp = lay.take<unsigned char>(tmp_bytes);
-  if(lay.off > kTrScratchBytes)
+  // the documented limit, 20 bytes per entry and 4 per column, is wider than the lists' 12 and 4
+  if(20 * nnz + 4 * cols > kTrScratchBytes)
     return fail(FEAT_ERR_UNSUPPORTED, "csr_apply_transposed_noalloc: the matrix needs more than the 32 MiB scratch "
-                                      "(about 20 bytes per entry and 4 per column)");
-  uint32_t* colptr = at(o_colptr);
-  if(nnz)
-  {
-    hipLaunchKernelGGL((k_tr_keys<IT>), dim3(grid_for(nnz, 4)), dim3(kThreads), 0, s, col, nnz, dk.Current(),
-                       dv.Current());
-    hipLaunchKernelGGL((k_tr_row_of<IT>), dim3(grid_for(rows)), dim3(kThreads), 0, s, rowptr, rows, at(o_row));
-    int rc = check_launch(name);
-    if(!rc)
-      rc = check_hip(hipcub::DeviceRadixSort::SortPairs(static_cast<void*>(base + o_tmp), tmp_bytes, dk, dv, int(nnz), 0,
-                                                        end_bit, s),
-                     "transposed apply: sort");
-    if(rc) return rc;
-  }
-  hipLaunchKernelGGL(k_tr_colptr, dim3(grid_for(nnz + 1, 4)), dim3(kThreads), 0, s, dk.Current(), nnz, cols, colptr);
-  hipLaunchKernelGGL((k_tr_gather<DT>), dim3(grid_for(cols)), dim3(kThreads), 0, s, r, a, DT(b / a), x, y, int(bzero), val,
-                     colptr, dv.Current(), at(o_row), cols);
-  return check_launch(name);
+                                      "(20 bytes per entry and 4 per column)");
+  const TrLayout L(cols, nnz);
+  if(L.bytes > kTrScratchBytes)
+    return fail(FEAT_ERR_UNSUPPORTED, "csr_apply_transposed_noalloc: the matrix needs more than the 32 MiB scratch");
+  return tr_apply(h->stream, base, L, r, a, x, b, bzero, y, val, col, rowptr, rows, cols, nnz, name);
 }
 
 template int csr_apply_transposed_noalloc<double, uint64_t>(feat_handle_t, double*, double, const double*, double, bool,
                                                             const double*, const double*, const uint64_t*,
                                                             const uint64_t*, uint64_t, uint64_t, uint64_t, const char*);
+
+// the handle's pool, made at its first use
+static int pool_of(feat_handle_t h, hipMemPool_t* pool)
+{
+  std::lock_guard<std::mutex> lk(h->pool_mutex);
+  if(!h->pool)
+  {
+    hipMemPoolProps props = {};
+    props.allocType = hipMemAllocationTypePinned;
+    props.handleTypes = hipMemHandleTypeNone;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = h->device;
+    hipMemPool_t p = nullptr;
+    int rc = check_hip(hipMemPoolCreate(&p, &props), "transposed apply: pool");
+    if(rc) return rc;
+    uint64_t keep = kTrPoolBytes;
+    rc = check_hip(hipMemPoolSetAttribute(p, hipMemPoolAttrReleaseThreshold, &keep), "transposed apply: pool");
+    if(rc)
+    {
+      (void)hipMemPoolDestroy(p);
+      return rc;
+    }
+    h->pool = p;
+  }
+  *pool = h->pool;
+  return FEAT_OK;
+}
 
 template<typename DT, typename IT>
 int csr_apply_transposed(feat_handle_t h, DT* r, DT a, const DT* x, DT b, bool bzero, const DT* y, const DT* val,
@@ -181,47 +474,14 @@ int csr_apply_transposed(feat_handle_t h, DT* r, DT a, const DT* x, DT b, bool b
   if(nnz >= (uint64_t(1) << 31) || rows >= (uint64_t(1) << 32) || cols >= (uint64_t(1) << 32))
     return fail(FEAT_ERR_UNSUPPORTED, "csr_apply: transposed apply needs fewer than 2^31 entries and 2^32 rows, columns");
   if(!cols) return FEAT_OK;
-  hipStream_t s = h->stream;
-  uint32_t *keys = nullptr, *keys_s = nullptr, *idx = nullptr, *order = nullptr, *row_of = nullptr, *colptr = nullptr;
-  void* tmp = nullptr;
-  size_t tmp_bytes = 0;
-  int end_bit = 1;
-  while(end_bit < 32 && (uint64_t(1) << end_bit) < cols) ++end_bit;
-  int rc = FEAT_OK;
-  auto release = [&]() {
-    for(void* p : {(void*)keys, (void*)keys_s, (void*)idx, (void*)order, (void*)row_of, (void*)colptr, tmp})
-      if(p) (void)hipFreeAsync(p, s);
-  };
-  rc = dev_alloc(&colptr, cols + 1, s);
-  if(!rc && nnz)
-  {
-    rc = dev_alloc(&keys, nnz, s);
-    if(!rc) rc = dev_alloc(&keys_s, nnz, s);
-    if(!rc) rc = dev_alloc(&idx, nnz, s);
-    if(!rc) rc = dev_alloc(&order, nnz, s);
-    if(!rc) rc = dev_alloc(&row_of, nnz, s);
-    if(!rc)
-      rc = check_hip(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp_bytes, keys, keys_s, idx, order, int(nnz), 0, end_bit, s),
-                     "transposed apply: sort size");
-    if(!rc) rc = check_hip(hipMallocAsync(&tmp, tmp_bytes ? tmp_bytes : 1, s), "transposed apply: sort buffer");
-    if(!rc)
-    {
-      hipLaunchKernelGGL((k_tr_keys<IT>), dim3(grid_for(nnz, 4)), dim3(kThreads), 0, s, col, nnz, keys, idx);
-      hipLaunchKernelGGL((k_tr_row_of<IT>), dim3(grid_for(rows)), dim3(kThreads), 0, s, rowptr, rows, row_of);
-      rc = check_launch(name);
-    }
-    if(!rc)
-      rc = check_hip(hipcub::DeviceRadixSort::SortPairs(tmp, tmp_bytes, keys, keys_s, idx, order, int(nnz), 0, end_bit, s),
-                     "transposed apply: sort");
-  }
-  if(!rc)
-  {
-    hipLaunchKernelGGL(k_tr_colptr, dim3(grid_for(nnz + 1, 4)), dim3(kThreads), 0, s, keys_s, nnz, cols, colptr);
-    hipLaunchKernelGGL((k_tr_gather<DT>), dim3(grid_for(cols)), dim3(kThreads), 0, s, r, a, DT(b / a), x, y, int(bzero),
-                       val, colptr, order, row_of, cols);
-    rc = check_launch(name);
-  }
-  release();
+  const TrLayout L(cols, nnz);
+  hipMemPool_t pool = nullptr;
+  void* base = nullptr;
+  int rc = pool_of(h, &pool);
+  if(!rc) rc = check_hip(hipMallocFromPoolAsync(&base, L.bytes, pool, h->stream), "transposed apply: buffer");
+  if(rc) return rc;
+  rc = tr_apply(h->stream, static_cast<unsigned char*>(base), L, r, a, x, b, bzero, y, val, col, rowptr, rows, cols, nnz, name);
+  (void)hipFreeAsync(base, h->stream);
   return rc;
 }
 

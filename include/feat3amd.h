@@ -100,8 +100,9 @@ int feat_convert_u64_u32(feat_handle_t h, uint32_t* dst, const uint64_t* src, ui
  * (bit-identical to the sequential CPU loop); the transposed form computes
  * (b/a)*y, adds each column's entries in ascending entry order (the order of the
  * generic row-by-row scatter) and scales by a: bit-identical too.  The
- * transposed form allocates stream-ordered sort buffers (about 20 bytes per
- * entry) in each call and needs nnz < 2^31; it is not for recorded graphs. */
+ * transposed form takes stream-ordered buffers for the column lists (about 12 bytes per
+ * entry) from a pool of the handle's (which keeps up to 256 MiB between calls) and needs
+ * nnz < 2^31; it is not for recorded graphs. */
 int feat_csr_apply_f64_u64(feat_handle_t h, double* r, double a, const double* x, double b,
                            const double* y, const double* val, const uint64_t* col,
                            const uint64_t* rowptr, uint64_t rows, uint64_t cols, uint64_t nnz,
@@ -121,10 +122,10 @@ int feat_csr_apply_f32_u64(feat_handle_t h, float* r, float a, const float* x, f
 
 /* The transposed form of feat_csr_apply_f64_u64 (transposed != 0) without any allocation:
  * no counterpart in the reference.  It is for callers that cannot allocate device memory
- * in the call (HIP graph capture, serving loops, harnesses that forbid it).  Its sort
- * buffers live in a static device array of FEAT_TR_NOALLOC_SCRATCH_BYTES per GPU, held
- * until the process ends and looked up when a handle is created; a matrix needing more
- * (about 20 bytes per entry plus 4 per column and the sort's own few KB) is rejected with
+ * in the call (HIP graph capture, serving loops, harnesses that forbid it).  Its column
+ * lists live in a static device array of FEAT_TR_NOALLOC_SCRATCH_BYTES per GPU, held
+ * until the process ends and looked up when a handle is created; a matrix of more than
+ * 20 bytes per entry plus 4 per column of it is rejected with
  * FEAT_ERR_UNSUPPORTED before anything runs.  Same arithmetic, bit-identical results.
  * Calls that overlap on one GPU (any handle, any stream) share that array and race. */
 #define FEAT_TR_NOALLOC_SCRATCH_BYTES (32u << 20)
