@@ -41,8 +41,7 @@ constexpr int kThreads = 256;
 constexpr int kXcd = 8;
 constexpr int kMaxGrid = FEAT_REDUCE_MAX_BLOCKS;
 constexpr int kRowsPerBlock = 256;  // rows per CSR row-block (one lane per row)
-constexpr int kCsrUnroll = 4;       // CSR entries each thread loads per pass
-constexpr int kChunk = kCsrUnroll * kThreads;   // nonzeros staged in LDS per pass
+constexpr uint64_t kCsrStream = 6144;   // CSR row-blocks from which a matrix streams from HBM
 constexpr int kSellUnroll = 8;      // SELL entries per row in flight
 
 

@@ -3,10 +3,10 @@
 // Design (MI355X / CDNA4):
 //  * CSR SpMV: rows are processed in row-blocks of kRowsPerBlock (256, one lane
 //    per row).  A 256-thread workgroup streams the contiguous nonzero range of its
-//    row-block through LDS in passes of kChunk entries (val and the gathered
-//    x[col] side by side, fully coalesced 64-wide loads, all of a pass in flight
-//    before the first store), then each lane sums its row's entries from LDS in
-//    storage order with one fma per entry.  The per-row arithmetic is therefore exactly the
+//    row-block through LDS in passes of 1024 or 2048 entries (val and the gathered
+//    x[col] side by side, fully coalesced 64-wide loads, two passes ahead), and
+//    each lane sums its row's entries from LDS in storage order with one fma per
+//    entry.  The per-row arithmetic is therefore exactly the
 //    reference's sequential loop (arch/apply_generic.hpp:57-66), bit for bit,
 //    while HBM sees only coalesced streams.  Fused epilogues apply the unit
 //    filter (bit mask), the defect/Richardson/Jacobi updates and reductions.
@@ -87,22 +87,31 @@ struct EpiCentre<E, DT, std::void_t<decltype(std::declval<const E&>().pre(uint64
 // ---------------------------------------------------------------------------
 // CSR row-block kernel with a fused epilogue.
 //   Epi::row(row, sum, acc0, acc1) is called once per row by its lane.
+//
+// The passes of a row-block are pipelined: while the lanes add up pass p from LDS (two buffers,
+// one barrier a pass), the gathers of pass p + 1 and the values and columns of pass p + 2 are
+// in flight.  One pass after the other (load, gather, store, barrier, add, barrier) a block of
+// ragged rows was one long chain of round trips: 300 k rows of 0 to 40 entries, FP32, 31 us;
+// now 26 us, bound by the 64 cache lines of each scattered gather.  50 k such rows 22.7 -> 9 us
+// (FP64, 64-bit columns 19.5 -> 12), 3D Q1 level 5 18.6 -> 11.4 us; level 7, which streams 982 MB
+// at the rate of a copy, does without (PIPE false; launch_rows).
 // ---------------------------------------------------------------------------
-template<typename DT, typename IT, class Epi>
+template<typename DT, typename IT, class Epi, int U, bool PIPE>
 __global__ __launch_bounds__(kThreads) void k_csr_rows(const DT* __restrict__ val,
                                                        const IT* __restrict__ col,
                                                        const IT* __restrict__ rowptr,
                                                        const DT* __restrict__ x, uint64_t rows,
                                                        Epi epi, GridReduce gr)
 {
-  static_assert(kChunk == kCsrUnroll * kThreads, "one pass = kCsrUnroll entries per thread");
-  __shared__ DT s_val[kChunk];
-  __shared__ DT s_x[kChunk];
+  constexpr uint32_t C = U * kThreads;   // entries a pass
+  __shared__ DT s_val[PIPE ? 2 : 1][C];
+  __shared__ DT s_x[PIPE ? 2 : 1][C];
   const uint64_t nrb = (rows + kRowsPerBlock - 1) / kRowsPerBlock;
   const XcdRange xr = xcd_range(nrb);
   const int t = threadIdx.x;
   double acc0 = 0.0, acc1 = 0.0;
   epi.begin();
+  int buf = 0;
   for(uint64_t rb = xr.first; rb < xr.end; rb += xr.stride)
   {
     const uint64_t r0 = rb * kRowsPerBlock;
@@ -119,39 +128,107 @@ __global__ __launch_bounds__(kThreads) void k_csr_rows(const DT* __restrict__ va
       if constexpr(EpiPre<Epi>::on) pf = epi.pre(r0 + t);
     }
     DT sum = DT(0);
-    for(uint64_t c0 = p0; c0 < p1; c0 += kChunk)
+    // the lane's entries of the pass at c0, from buffer b
+    auto add = [&](uint64_t c0, int b) {
+      if(!mine) return;
+      const uint64_t ce = c0 + C < p1 ? c0 + C : p1;
+      const uint64_t kb = rs > c0 ? rs : c0;
+      const uint64_t ke = re < ce ? re : ce;
+      if(kb >= ke) return;
+      const DT* sv = &s_val[b][kb - c0];
+      const DT* sx = &s_x[b][kb - c0];
+      const int n = int(ke - kb);
+#pragma unroll 4
+      for(int k = 0; k < n; ++k) sum = dfma(sv[k], sx[k], sum);
+    };
+    if constexpr(!PIPE)
     {
-      const uint64_t cn = (p1 - c0) < uint64_t(kChunk) ? (p1 - c0) : uint64_t(kChunk);
-      // every value and column of the pass is requested before the first gather of x,
-      // and every gather before the first LDS store (the matrix is streamed once:
-      // nontemporal loads keep x resident in L2)
-      DT v[kCsrUnroll], xv[kCsrUnroll];
-      uint64_t cc[kCsrUnroll];
-#pragma unroll
-      for(int u = 0; u < kCsrUnroll; ++u)
+      for(uint64_t c0 = p0; c0 < p1; c0 += C)
       {
-        const uint64_t j = uint64_t(t) + uint64_t(u) * kThreads;
-        v[u] = j < cn ? __builtin_nontemporal_load(val + c0 + j) : DT(0);
-        cc[u] = j < cn ? uint64_t(__builtin_nontemporal_load(col + c0 + j)) : 0;
-      }
+        const uint64_t cn = (p1 - c0) < uint64_t(C) ? (p1 - c0) : uint64_t(C);
+        // every value and column of the pass is requested before the first gather of x, and
+        // every gather before the first LDS store
+        DT v[U], xv[U];
+        uint64_t cc[U];
 #pragma unroll
-      for(int u = 0; u < kCsrUnroll; ++u)
-        xv[u] = uint64_t(t) + uint64_t(u) * kThreads < cn ? x[cc[u]] : DT(0);
+        for(int u = 0; u < U; ++u)
+        {
+          const uint64_t j = uint64_t(t) + uint64_t(u) * kThreads;
+          v[u] = j < cn ? __builtin_nontemporal_load(val + c0 + j) : DT(0);
+          cc[u] = j < cn ? uint64_t(__builtin_nontemporal_load(col + c0 + j)) : 0;
+        }
 #pragma unroll
-      for(int u = 0; u < kCsrUnroll; ++u)
-      {
-        s_val[t + u * kThreads] = v[u];
-        s_x[t + u * kThreads] = xv[u];
+        for(int u = 0; u < U; ++u) xv[u] = uint64_t(t) + uint64_t(u) * kThreads < cn ? x[cc[u]] : DT(0);
+#pragma unroll
+        for(int u = 0; u < U; ++u)
+        {
+          s_val[0][t + u * kThreads] = v[u];
+          s_x[0][t + u * kThreads] = xv[u];
+        }
+        __syncthreads();
+        add(c0, 0);
+        __syncthreads();
       }
-      __syncthreads();
-      if(mine)
+    }
+    else if(p0 < p1)
+    {
+      // every load is unconditional (positions past the block's end read its last entry and are
+      // not added) and the two register sets take turns, so that no wait covers the loads of a
+      // later pass.  The matrix is streamed once: nontemporal loads keep x resident in L2.
+      struct Pass
       {
-        const uint64_t kb = rs > c0 ? rs : c0;
-        const uint64_t ke = re < c0 + cn ? re : c0 + cn;
-        for(uint64_t k = kb; k < ke; ++k)
-          sum = dfma(s_val[k - c0], s_x[k - c0], sum);
+        DT v[U], xv[U];
+        IT c[U];
+      };
+      auto fetch = [&](uint64_t c0, Pass& a) {
+#pragma unroll
+        for(int u = 0; u < U; ++u)
+        {
+          const uint64_t k = c0 + uint64_t(t + u * kThreads);
+          a.c[u] = __builtin_nontemporal_load(col + (k < p1 ? k : p1 - 1));
+        }
+#pragma unroll
+        for(int u = 0; u < U; ++u)
+        {
+          const uint64_t k = c0 + uint64_t(t + u * kThreads);
+          a.v[u] = __builtin_nontemporal_load(val + (k < p1 ? k : p1 - 1));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto gather = [&](Pass& a) {
+#pragma unroll
+        for(int u = 0; u < U; ++u) a.xv[u] = x[uint64_t(a.c[u])];
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      uint64_t c0 = p0;
+      auto step = [&](Pass& a, Pass& b) {
+#pragma unroll
+        for(int u = 0; u < U; ++u)
+        {
+          s_val[buf][t + u * kThreads] = a.v[u];
+          s_x[buf][t + u * kThreads] = a.xv[u];
+        }
+        // a wave that is here has added up the pass before the last one, whose buffer the next
+        // pass takes once all waves have passed
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        gather(b);
+        fetch(c0 + 2 * C, a);
+        add(c0, buf);
+        c0 += C;
+        buf ^= 1;
+      };
+      Pass a, b;
+      fetch(p0, a);
+      gather(a);
+      fetch(p0 + C, b);
+      while(c0 < p1)
+      {
+        step(a, b);
+        if(c0 >= p1) break;
+        step(b, a);
       }
-      __syncthreads();
     }
     if(mine)
     {
@@ -368,8 +445,15 @@ int launch_rows(hipStream_t s, const DT* val, const IT* col, const IT* rowptr, c
   const uint64_t nrb = (rows + kRowsPerBlock - 1) / kRowsPerBlock;
   const int grid = int(nrb < uint64_t(kMaxGrid) ? nrb : uint64_t(kMaxGrid));
   const GridReduce gd = reduce_for_grid(gr, uint64_t(grid));
-  hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi>), dim3(grid), dim3(kThreads), 0, s, val, col, rowptr,
-                     x, rows, epi, gd);
+  // a matrix of 8-byte values that fills the chip many times over streams at the rate of a copy
+  // without the pipeline, whose loads past a block's end cost it 2 % (3D Q1 level 7, 8386
+  // row-blocks: 193 against 197 us; 4-byte values, and 5000 blocks: the pipeline, 92 against 111 us)
+  if(sizeof(DT) == 8 && nrb >= kCsrStream)
+    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 4, false>), dim3(grid), dim3(kThreads), 0, s, val, col, rowptr, x, rows, epi,
+                       gd);
+  else
+    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 32 / int(sizeof(DT)), true>), dim3(grid), dim3(kThreads), 0, s, val, col,
+                       rowptr, x, rows, epi, gd);
   finish_reduce(s, gd, uint64_t(grid));
   return check_launch(name);
 }

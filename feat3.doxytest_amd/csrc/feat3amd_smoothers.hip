@@ -325,12 +325,12 @@ int build_chain(const std::vector<uint64_t>& off, const std::vector<uint32_t>& p
   if(slots >= (uint64_t(1) << 32) || 64 * slots > kChainSlotsPerLevel * nl) return FEAT_OK;
   std::vector<uint16_t> len(64 * ns, 0);
   std::vector<uint32_t> row(64 * ns, kNoRow), src(64 * words, kRing | (kRing << 16));
-  std::vector<uint64_t> map(64 * slots, kNoEntry), cmap(64 * ns, kNoEntry);
+  std::vector<uint64_t> map(64 * slots, kNoEntry), cmap(csrc(0) == kNoEntry ? 1 : 64 * ns, kNoEntry);
   for(uint64_t r = 0; r < n; ++r)
   {
     const uint64_t p = pos[r], s = p / 64, lane = p % 64;
     row[p] = uint32_t(r);
-    cmap[p] = csrc(r);
+    if(cmap.size() > 1) cmap[p] = csrc(r);
     uint32_t t = 0;
     for(uint64_t k = begin(r); k != end(r); k += uint64_t(std::int64_t(step)), ++t)
     {
@@ -963,6 +963,10 @@ int feat_ilu_init_symbolic_p(feat_handle_t h, const feat_csr_f64_t* A, int p, fe
   // L / D / U split (set_struct_csr: every row needs its diagonal entry)
   std::vector<uint64_t> rl{0}, ru{0}, ml, mu, md(n);
   std::vector<uint32_t> cl, cu;
+  rl.reserve(n + 1);
+  ru.reserve(n + 1);
+  for(auto* v : {&ml, &mu}) v->reserve(nnz / 2 + n);
+  for(auto* v : {&cl, &cu}) v->reserve(nnz / 2 + n);
   for(uint64_t i = 0; i < n; ++i)
   {
     bool diag = false;
