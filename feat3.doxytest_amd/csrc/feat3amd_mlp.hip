@@ -7,9 +7,8 @@
 // are staged in LDS; the 16x16 MFMA lane layout is
 //   A: lane l holds A[l%16][k0 + 4*(l/16) + i], B: B[k0 + 4*(l/16) + i][l%16],
 //   D: lane l holds D[4*(l/16) + i][l%16], i = 0..3.
-// Per-sample and per-unit sums outside the MFMAs (layer 3, bias and layer-3
-// gradients, the loss) run sequentially in a fixed order, and weight gradients
-// are reduced over wavefronts in index order: training is deterministic.
+// Sums outside the MFMAs (layer 3, bias and layer-3 gradients, the loss) and the reduction
+// of the weight gradients over wavefronts run in a fixed order: training is deterministic.
 #include "feat3amd_common.hpp"
 
 namespace {
@@ -27,8 +26,6 @@ __device__ __forceinline__ uint16_t f2bf(float f)
   // round to nearest even: gfx950's v_cvt_pk_bf16_f32
   return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float(uint32_t(b) << 16); }
-__device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
 // GELU of the inference kernels: erf by Abramowitz & Stegun 7.1.26 (|error| <= 1.5e-7,
 // far below the BF16 rounding its result goes through), one reciprocal and one exp
 __device__ __forceinline__ float gelu_fast(float z)
@@ -43,215 +40,6 @@ __device__ __forceinline__ float gelu_fast(float z)
   const float e = 1.0f - p * t * __expf(-x * x);
   return 0.5f * z * (1.0f + copysignf(e, z));
 }
-__device__ __forceinline__ float gelu_d(float z)
-{
-  return 0.5f * (1.0f + erff(z * 0.70710678118654752f)) + z * 0.39894228040143268f * expf(-0.5f * z * z);
-}
-
-// acc += A(16 x K) * B(K x 16), A(m,k) = A[m*ars + k*acs], B(k,n) = B[k*brs + n*bcs], BF16 in LDS
-__device__ __forceinline__ f32x4 mfma_tile(f32x4 acc, const uint16_t* A, int ars, int acs, const uint16_t* B, int brs,
-                                           int bcs, int K)
-{
-  const int l = threadIdx.x & 63, r = l & 15, kq = (l >> 4) * 4;
-  for(int k0 = 0; k0 < K; k0 += 16)
-  {
-    bf16x4 a, b;
-#pragma unroll
-    for(int i = 0; i < 4; ++i)
-    {
-      a[i] = short(A[r * ars + (k0 + kq + i) * acs]);
-      b[i] = short(B[(k0 + kq + i) * brs + r * bcs]);
-    }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-  }
-  return acc;
-}
-
-struct SharedWeights
-{
-  uint16_t w1[kHid * kInP];
-  uint16_t w2[kHid * kHid];
-  float b1[kHid], b2[kHid], w3[kHid];
-  float b3;
-};
-
-__device__ void load_weights(SharedWeights& W, const float* __restrict__ p, const uint16_t* __restrict__ wbf)
-{
-  for(int i = threadIdx.x; i < kHid * kInP; i += blockDim.x)
-  {
-    W.w1[i] = wbf[i];
-    W.w2[i] = wbf[kHid * kInP + i];
-  }
-  for(int i = threadIdx.x; i < kHid; i += blockDim.x)
-  {
-    W.b1[i] = p[kB1 + i];
-    W.b2[i] = p[kB2 + i];
-    W.w3[i] = p[kW3 + i];
-  }
-  if(threadIdx.x == 0) W.b3 = p[kB3];
-}
-
-struct WaveBuf
-{
-  uint16_t x[16 * kInP];
-  uint16_t h1[16 * kHid];
-  float z1[16 * kHid];
-  float z2[16 * kHid];
-  uint16_t d2[16 * kHid];
-  uint16_t d1[16 * kHid];
-  float y[16];
-};
-
-// layers 1 and 2 for the wave's 16 samples in B.x: fills z1, h1, z2 (LDS); returns nothing
-__device__ void forward12(const SharedWeights& W, WaveBuf& B)
-{
-  const int l = threadIdx.x & 63, r = l & 15, kq = (l >> 4) * 4;
-  for(int nt = 0; nt < 4; ++nt)
-  {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma_tile(acc, B.x, kInP, 1, W.w1 + nt * 16 * kInP, 1, kInP, kInP);
-#pragma unroll
-    for(int i = 0; i < 4; ++i) B.z1[(kq + i) * kHid + nt * 16 + r] = acc[i] + W.b1[nt * 16 + r];
-  }
-  __syncthreads();
-  for(int e = l; e < 16 * kHid; e += 64) B.h1[e] = f2bf(gelu(B.z1[e]));
-  __syncthreads();
-  for(int nt = 0; nt < 4; ++nt)
-  {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma_tile(acc, B.h1, kHid, 1, W.w2 + nt * 16 * kHid, 1, kHid, kHid);
-#pragma unroll
-    for(int i = 0; i < 4; ++i) B.z2[(kq + i) * kHid + nt * 16 + r] = acc[i] + W.b2[nt * 16 + r];
-  }
-  __syncthreads();
-  // layer 3 in FP32: y = b3 + sum_o w3[o] gelu(z2[o]), sequential in o
-  if(l < 16)
-  {
-    float y = 0.0f;
-    for(int o = 0; o < kHid; ++o) y = __fmaf_rn(W.w3[o], gelu(B.z2[l * kHid + o]), y);
-    B.y[l] = y + W.b3;
-  }
-  __syncthreads();
-}
-
-// Training: forward + backward over tiles of 64 samples per workgroup; per-wave
-// gradient partials (FEAT_MLP_NPARAM_PAD floats each, loss in the last slot).
-__global__ __launch_bounds__(64 * kWaves) void k_mlp_train(const float* __restrict__ p, const uint16_t* __restrict__ wbf,
-                                                           const uint16_t* __restrict__ X, const float* __restrict__ t,
-                                                           uint64_t nsamp, float inv_b, float* __restrict__ partials)
-{
-  __shared__ SharedWeights W;
-  __shared__ WaveBuf Bw[kWaves];
-  __shared__ float gb1[kWaves][kHid], gb2[kWaves][kHid], gw3[kWaves][kHid], gb3[kWaves], gloss[kWaves];
-  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 15, kq = (l >> 4) * 4;
-  WaveBuf& B = Bw[wave];
-  load_weights(W, p, wbf);
-  gb1[wave][l] = gb2[wave][l] = gw3[wave][l] = 0.0f;
-  if(l == 0) gb3[wave] = gloss[wave] = 0.0f;
-  f32x4 aw1[4][4], aw2[4][4];
-  for(int a = 0; a < 4; ++a)
-    for(int b = 0; b < 4; ++b) aw1[a][b] = aw2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  __syncthreads();
-  const uint64_t ngroups = (nsamp + 16 * kWaves - 1) / (16 * kWaves);
-  for(uint64_t g = blockIdx.x; g < ngroups; g += gridDim.x)
-  {
-    const uint64_t s0 = (g * kWaves + uint64_t(wave)) * 16;
-    for(int e = l; e < 16 * kInP; e += 64)
-    {
-      const uint64_t s = s0 + uint64_t(e / kInP);
-      B.x[e] = s < nsamp ? X[s * kInP + uint64_t(e % kInP)] : uint16_t(0);
-    }
-    __syncthreads();
-    forward12(W, B);
-    // dy, loss, layer-3 gradients: lane o walks the 16 samples in order
-    __shared__ float dyv[kWaves][16];
-    if(l < 16)
-    {
-      const uint64_t s = s0 + uint64_t(l);
-      float dy = 0.0f;
-      if(s < nsamp)
-      {
-        const float d = B.y[l] - t[s];
-        dy = 2.0f * d * inv_b;
-      }
-      dyv[wave][l] = dy;
-    }
-    __syncthreads();
-    if(l == 0)
-      for(int s = 0; s < 16; ++s)
-        if(s0 + uint64_t(s) < nsamp)
-        {
-          const float d = B.y[s] - t[s0 + uint64_t(s)];
-          gloss[wave] = __fmaf_rn(d, d, gloss[wave]);
-          gb3[wave] += dyv[wave][s];
-        }
-    {
-      const int o = l;
-      float a2 = gb2[wave][o], a3 = gw3[wave][o];
-      for(int s = 0; s < 16; ++s)
-      {
-        const float z = B.z2[s * kHid + o], dy = dyv[wave][s];
-        const float dz2 = dy * W.w3[o] * gelu_d(z);
-        a3 = __fmaf_rn(dy, gelu(z), a3);
-        a2 += dz2;
-        B.d2[s * kHid + o] = f2bf(dz2);
-      }
-      gb2[wave][o] = a2;
-      gw3[wave][o] = a3;
-    }
-    __syncthreads();
-    // dW2 += dZ2^T H1 (M = out unit, N = in unit, K = samples)
-    for(int mt = 0; mt < 4; ++mt)
-      for(int nt = 0; nt < 4; ++nt)
-        aw2[mt][nt] = mfma_tile(aw2[mt][nt], B.d2 + mt * 16, 1, kHid, B.h1 + nt * 16, kHid, 1, 16);
-    // dH1 = dZ2 W2, dZ1 = dH1 * gelu'(Z1) (stored FP32 in z2's place, BF16 in d1)
-    for(int nt = 0; nt < 4; ++nt)
-    {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-      acc = mfma_tile(acc, B.d2, kHid, 1, W.w2 + nt * 16, kHid, 1, kHid);
-#pragma unroll
-      for(int i = 0; i < 4; ++i)
-      {
-        const int e = (kq + i) * kHid + nt * 16 + r;
-        const float dz1 = acc[i] * gelu_d(B.z1[e]);
-        B.z2[e] = dz1;
-        B.d1[e] = f2bf(dz1);
-      }
-    }
-    __syncthreads();
-    {
-      const int o = l;
-      float a1 = gb1[wave][o];
-      for(int s = 0; s < 16; ++s) a1 += B.z2[s * kHid + o];
-      gb1[wave][o] = a1;
-    }
-    // dW1 += dZ1^T X
-    for(int mt = 0; mt < 4; ++mt)
-      for(int nt = 0; nt < 4; ++nt)
-        aw1[mt][nt] = mfma_tile(aw1[mt][nt], B.d1 + mt * 16, 1, kHid, B.x + nt * 16, kInP, 1, 16);
-    __syncthreads();
-  }
-  float* out = partials + (uint64_t(blockIdx.x) * kWaves + uint64_t(wave)) * FEAT_MLP_NPARAM_PAD;
-  for(int mt = 0; mt < 4; ++mt)
-    for(int nt = 0; nt < 4; ++nt)
-#pragma unroll
-      for(int i = 0; i < 4; ++i)
-      {
-        const int row = mt * 16 + kq + i, col = nt * 16 + r;
-        out[kW1 + row * kInP + col] = aw1[mt][nt][i];
-        out[kW2 + row * kHid + col] = aw2[mt][nt][i];
-      }
-  out[kB1 + l] = gb1[wave][l];
-  out[kB2 + l] = gb2[wave][l];
-  out[kW3 + l] = gw3[wave][l];
-  if(l == 0)
-  {
-    out[kB3] = gb3[wave];
-    out[kLoss] = gloss[wave];
-  }
-  for(int i = kB3 + 1 + l; i < kLoss; i += 64) out[i] = 0.0f;
-}
-
 // Gradient reduction in a fixed order: segment g sums partial vectors 32g .. 32g+31 in
 // index order (stage 0), then grad[i] sums the segments in index order (stage 1);
 // padded inputs get no gradient.
@@ -262,7 +50,15 @@ __global__ void k_mlp_reduce_seg(const float* __restrict__ partials, uint64_t np
   if(i >= uint64_t(FEAT_MLP_NPARAM_PAD)) return;
   const uint64_t w0 = uint64_t(blockIdx.y) * kRedSeg, w1 = w0 + kRedSeg < nparts ? w0 + kRedSeg : nparts;
   float s = 0.0f;
-  for(uint64_t w = w0; w < w1; ++w) s += partials[w * FEAT_MLP_NPARAM_PAD + i];
+  for(uint64_t wb = w0; wb < w1; wb += 16)   // 16 loads in flight, added in order
+  {
+    float v[16];
+#pragma unroll
+    for(int u = 0; u < 16; ++u) v[u] = partials[(wb + u < w1 ? wb + u : w1 - 1) * FEAT_MLP_NPARAM_PAD + i];
+#pragma unroll
+    for(int u = 0; u < 16; ++u)
+      if(wb + u < w1) s += v[u];
+  }
   seg[uint64_t(blockIdx.y) * FEAT_MLP_NPARAM_PAD + i] = s;
 }
 __global__ void k_mlp_reduce(const float* __restrict__ seg, uint64_t nseg, float* __restrict__ grad)
@@ -270,7 +66,15 @@ __global__ void k_mlp_reduce(const float* __restrict__ seg, uint64_t nseg, float
   const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if(i >= uint64_t(FEAT_MLP_NPARAM_PAD)) return;
   float s = 0.0f;
-  for(uint64_t w = 0; w < nseg; ++w) s += seg[w * FEAT_MLP_NPARAM_PAD + i];
+  for(uint64_t wb = 0; wb < nseg; wb += 16)
+  {
+    float v[16];
+#pragma unroll
+    for(int u = 0; u < 16; ++u) v[u] = seg[(wb + u < nseg ? wb + u : nseg - 1) * FEAT_MLP_NPARAM_PAD + i];
+#pragma unroll
+    for(int u = 0; u < 16; ++u)
+      if(wb + u < nseg) s += v[u];
+  }
   if(i < uint64_t(kB1) && (i % kInP) >= uint64_t(kIn)) s = 0.0f;
   grad[i] = s;
 }
@@ -368,6 +172,274 @@ __device__ __forceinline__ float forward_t(const LdsWeights& W, const bf16x4 (&X
   part += __shfl_xor(part, 16, 64);
   part += __shfl_xor(part, 32, 64);
   return part + W.b3;
+}
+
+// Weights of the training kernel: the fragments of W1 and W2 as above, and those of W2^T for
+// the way back (fragment (mt, ks) of lane l = W2[ks*16 + 4(l/16) + i][mt*16 + l%16]).
+struct TrainWeights
+{
+  LdsWeights f;
+  bf16x4 w2t[16 * 64];
+};
+
+constexpr int kTStride = 20;   // samples of a transposed row, padded (8-byte aligned reads)
+// bf16 values of 64 units x 16 samples of one wavefront, unit-major
+struct TransTile
+{
+  uint16_t v[kHid * kTStride];
+  // lane l holds units nt*16 + 4(l/16) + i of sample l%16 (the layout forward_t works in)
+  __device__ __forceinline__ void put(const bf16x4 (&f)[4])
+  {
+    const int l = threadIdx.x & 63, c = l & 15, q = l >> 4;
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for(int i = 0; i < 4; ++i) v[(nt * 16 + 4 * q + i) * kTStride + c] = uint16_t(f[nt][i]);
+  }
+  // operand with the samples as K: unit nt*16 + l%16, samples 4(l/16) + i
+  __device__ __forceinline__ bf16x4 get(int nt) const
+  {
+    const int l = threadIdx.x & 63, c = l & 15, q = l >> 4;
+    bf16x4 r;
+    __builtin_memcpy(&r, v + (nt * 16 + c) * kTStride + 4 * q, 8);
+    return r;
+  }
+};
+
+// GELU and its derivative from one erf(z / sqrt 2)
+__device__ __forceinline__ void gelu_both(float z, float& g, float& d)
+{
+  const float e = erff(z * 0.70710678118654752f);
+  g = 0.5f * z * (1.0f + e);
+  d = 0.5f * (1.0f + e) + z * 0.39894228040143268f * expf(-0.5f * z * z);
+}
+
+// Training: forward and backward of tiles of 16 samples a wavefront, one gradient vector
+// (FEAT_MLP_NPARAM_PAD floats, loss in the last slot) a workgroup.
+//
+// Everything stays in the transposed layout of forward_t (units x sample in registers), so both
+// layers and the way back (dH1^T = W2^T dZ2^T) take their operands straight from registers and
+// from weight fragments read 8 bytes at a time.  Only the weight gradients, whose products run
+// over the samples, need their four operands turned round through LDS.  erf is evaluated once a
+// unit.  (The form before it kept all activations in LDS, read its operands two bytes at a time
+// and evaluated erf twice.)  A workgroup adds its wavefronts' sums in order before it writes
+// them: a quarter of the gradient vectors to reduce.  feat_mlp_grad on 729 samples 41 -> 22 us,
+// on 35,937 112 -> 39 us, on 274,625 464 -> 122 us (23 TFLOP/s), bound by the erf and exp of
+// 128 units a sample.  330 registers leave one wave a SIMD; two, with 139 of them spilled, took
+// 65 us on 35,937 samples.
+__global__ __launch_bounds__(64 * kWaves) void k_mlp_train(const float* __restrict__ p, const uint16_t* __restrict__ wbf,
+                                                           const uint16_t* __restrict__ X, const float* __restrict__ t,
+                                                           uint64_t nsamp, float inv_b, float* __restrict__ partials)
+{
+  __shared__ TrainWeights W;
+  __shared__ union Tiles
+  {
+    TransTile t[kWaves][4];              // X, H1, dZ2, dZ1
+    float red[kWaves][2 * 4 * 4 * 64];   // a quarter of both weight gradients
+  } T;
+  __shared__ float vec[kWaves][3 * kHid + 2];
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, c = l & 15, q = l >> 4;
+  for(int f = threadIdx.x; f < 16 * 64; f += blockDim.x)
+  {
+    const int mt = f >> 8, ks = (f >> 6) & 3, fc = f & 15, fq = (f & 63) >> 4;
+    bf16x4 w;
+#pragma unroll
+    for(int i = 0; i < 4; ++i) w[i] = short(wbf[kHid * kInP + (ks * 16 + 4 * fq + i) * kHid + mt * 16 + fc]);
+    W.w2t[f] = w;
+  }
+  load_lds_weights(W.f, p, wbf);
+  f32x4 aw1[4][4], aw2[4][4];
+  float sb1[4][4], sb2[4][4], sw3[4][4], sb3 = 0.0f, loss = 0.0f;
+#pragma unroll
+  for(int a = 0; a < 4; ++a)
+#pragma unroll
+    for(int b = 0; b < 4; ++b)
+    {
+      aw1[a][b] = aw2[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+      sb1[a][b] = sb2[a][b] = sw3[a][b] = 0.0f;
+    }
+  const uint64_t ngroups = (nsamp + 16 * kWaves - 1) / (16 * kWaves);
+  for(uint64_t g = blockIdx.x; g < ngroups; g += gridDim.x)
+  {
+    asm volatile("" ::: "memory");
+    const uint64_t smp = (g * kWaves + uint64_t(wave)) * 16 + uint64_t(c);
+    const bool on = smp < nsamp;
+    const float target = on ? t[smp] : 0.0f;
+    bf16x4 Xo[4], H[4], D[4];
+#pragma unroll
+    for(int ks = 0; ks < 4; ++ks)
+    {
+      const bf16x4 v = *reinterpret_cast<const bf16x4*>(X + (on ? smp : 0) * kInP + ks * 16 + 4 * q);
+      Xo[ks] = on ? v : bf16x4{0, 0, 0, 0};
+    }
+    float g1[4][4], g2[4][4], a2[4][4];
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+    {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for(int ks = 0; ks < 4; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.f.w1[(nt * 4 + ks) * 64 + l], Xo[ks], acc, 0, 0, 0);
+#pragma unroll
+      for(int i = 0; i < 4; ++i)
+      {
+        float h;
+        gelu_both(acc[i] + W.f.b1[nt * 16 + 4 * q + i], h, g1[nt][i]);
+        H[nt][i] = short(f2bf(h));
+      }
+    }
+    float part = 0.0f;
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+    {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for(int ks = 0; ks < 4; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.f.w2[(nt * 4 + ks) * 64 + l], H[ks], acc, 0, 0, 0);
+#pragma unroll
+      for(int i = 0; i < 4; ++i)
+      {
+        const int u = nt * 16 + 4 * q + i;
+        gelu_both(acc[i] + W.f.b2[u], a2[nt][i], g2[nt][i]);
+        part = __fmaf_rn(W.f.w3[u], a2[nt][i], part);
+      }
+    }
+    part += __shfl_xor(part, 16, 64);
+    part += __shfl_xor(part, 32, 64);
+    const float d = on ? part + W.f.b3 - target : 0.0f;
+    const float dy = 2.0f * d * inv_b;
+    if(q == 0)
+    {
+      loss = __fmaf_rn(d, d, loss);
+      sb3 += dy;
+    }
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for(int i = 0; i < 4; ++i)
+      {
+        const float dz2 = dy * W.f.w3[nt * 16 + 4 * q + i] * g2[nt][i];
+        sw3[nt][i] = __fmaf_rn(dy, a2[nt][i], sw3[nt][i]);
+        sb2[nt][i] += dz2;
+        D[nt][i] = short(f2bf(dz2));
+      }
+    TransTile* tt = T.t[wave];
+    tt[0].put(Xo);
+    tt[1].put(H);
+    tt[2].put(D);
+    // dZ1 = (W2^T dZ2) * gelu'(Z1)
+    bf16x4 D1[4];
+#pragma unroll
+    for(int mt = 0; mt < 4; ++mt)
+    {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for(int ks = 0; ks < 4; ++ks)
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(W.w2t[(mt * 4 + ks) * 64 + l], D[ks], acc, 0, 0, 0);
+#pragma unroll
+      for(int i = 0; i < 4; ++i)
+      {
+        const float dz1 = acc[i] * g1[mt][i];
+        sb1[mt][i] += dz1;
+        D1[mt][i] = short(f2bf(dz1));
+      }
+    }
+    tt[3].put(D1);
+    // the tiles belong to this wavefront; its LDS operations run in order
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+    // dW2 += dZ2^T H1, dW1 += dZ1^T X (M = out unit, N = in unit, K = samples)
+    bf16x4 A[4], B[4];
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+    {
+      A[nt] = tt[2].get(nt);
+      B[nt] = tt[1].get(nt);
+    }
+#pragma unroll
+    for(int mt = 0; mt < 4; ++mt)
+#pragma unroll
+      for(int nt = 0; nt < 4; ++nt)
+        aw2[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[mt], B[nt], aw2[mt][nt], 0, 0, 0);
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+    {
+      A[nt] = tt[3].get(nt);
+      B[nt] = tt[0].get(nt);
+    }
+#pragma unroll
+    for(int mt = 0; mt < 4; ++mt)
+#pragma unroll
+      for(int nt = 0; nt < 4; ++nt)
+        aw1[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(A[mt], B[nt], aw1[mt][nt], 0, 0, 0);
+  }
+  // sums over the 16 samples' lanes of the bias and layer-3 gradients, the loss
+#pragma unroll
+  for(int nt = 0; nt < 4; ++nt)
+#pragma unroll
+    for(int i = 0; i < 4; ++i)
+    {
+      float v1 = sb1[nt][i], v2 = sb2[nt][i], v3 = sw3[nt][i];
+#pragma unroll
+      for(int o = 1; o < 16; o <<= 1)
+      {
+        v1 += __shfl_xor(v1, o, 64);
+        v2 += __shfl_xor(v2, o, 64);
+        v3 += __shfl_xor(v3, o, 64);
+      }
+      if(c == 0)
+      {
+        const int u = nt * 16 + 4 * q + i;
+        vec[wave][u] = v1;
+        vec[wave][kHid + u] = v2;
+        vec[wave][2 * kHid + u] = v3;
+      }
+    }
+#pragma unroll
+  for(int o = 1; o < 16; o <<= 1)
+  {
+    sb3 += __shfl_xor(sb3, o, 64);
+    loss += __shfl_xor(loss, o, 64);
+  }
+  if(l == 0)
+  {
+    vec[wave][3 * kHid] = sb3;
+    vec[wave][3 * kHid + 1] = loss;
+  }
+  // the wavefronts' weight gradients, 16 rows of both matrices at a time, added in wave order
+  float* out = partials + uint64_t(blockIdx.x) * FEAT_MLP_NPARAM_PAD;
+#pragma unroll
+  for(int mt = 0; mt < 4; ++mt)
+  {
+    __syncthreads();
+#pragma unroll
+    for(int nt = 0; nt < 4; ++nt)
+#pragma unroll
+      for(int i = 0; i < 4; ++i)
+      {
+        T.red[wave][(nt * 4 + i) * 64 + l] = aw1[mt][nt][i];
+        T.red[wave][(16 + nt * 4 + i) * 64 + l] = aw2[mt][nt][i];
+      }
+    __syncthreads();
+    for(int e = threadIdx.x; e < 32 * 64; e += 64 * kWaves)
+    {
+      float v = T.red[0][e];
+#pragma unroll
+      for(int w = 1; w < kWaves; ++w) v += T.red[w][e];
+      const int el = e & 63, k = e >> 6, nt = (k >> 2) & 3, i = k & 3;
+      const int row = mt * 16 + 4 * (el >> 4) + i, col = nt * 16 + (el & 15);
+      out[(k < 16 ? kW1 : kW2) + row * kHid + col] = v;
+    }
+  }
+  for(int e = threadIdx.x; e < 3 * kHid + 2; e += 64 * kWaves)
+  {
+    float v = vec[0][e];
+#pragma unroll
+    for(int w = 1; w < kWaves; ++w) v += vec[w][e];
+    const int k = e / kHid, u = e % kHid;
+    out[k == 0 ? kB1 + u : k == 1 ? kB2 + u : k == 2 ? kW3 + u : u == 0 ? kB3 : kLoss] = v;
+  }
+  for(int i = kB3 + 1 + threadIdx.x; i < kLoss; i += 64 * kWaves) out[i] = 0.0f;
 }
 
 // Plain inference on given inputs (training, tests, evaluation): each lane loads its
@@ -636,11 +708,14 @@ int feat_mlp_grad(feat_handle_t h, const float* params, const uint16_t* wbf, con
 {
   if(!h || !params || !wbf || !X || !t || !partials || !grad || !nsamp)
     return fail(FEAT_ERR_INVALID, "feat_mlp_grad: bad argument");
-  // at most 256 workgroups (each strides over its sample groups): few partial vectors
+  // at most 256 workgroups (one a CU: their registers leave no room for a second; each strides
+  // over its sample groups), one gradient vector each
   const uint64_t ng = (nsamp + 16 * kWaves - 1) / (16 * kWaves);
   const int grid = int(ng < 256 ? ng : 256);
-  const uint64_t nparts = uint64_t(grid) * kWaves, nseg = (nparts + kRedSeg - 1) / kRedSeg;
-  if(nparts + nseg > partials_cap) return fail(FEAT_ERR_INVALID, "feat_mlp_grad: partials buffer too small");
+  const uint64_t nparts = uint64_t(grid), nseg = (nparts + kRedSeg - 1) / kRedSeg;
+  // the documented size, four vectors for each workgroup, is more than is used
+  const uint64_t need = 4 * uint64_t(grid);
+  if(need + (need + kRedSeg - 1) / kRedSeg > partials_cap) return fail(FEAT_ERR_INVALID, "feat_mlp_grad: partials buffer too small");
   float* seg = partials + nparts * FEAT_MLP_NPARAM_PAD;
   hipLaunchKernelGGL(k_mlp_train, dim3(grid), dim3(64 * kWaves), 0, h->stream, params, wbf, X, t, nsamp,
                      1.0f / float(nsamp), partials);
