@@ -3543,17 +3543,32 @@ struct TailBufs
 // for the whole V-cycle: the smoothing and defect sweeps then touch only LDS.
 constexpr int kTailSmoothed = FEAT_MG_TAIL_MAX_LEVELS - 1;
 
-template<typename DT>
+// MODE: how the smoothed levels hold their rows (one form for all of them).
+//  * kTailPlan: FEAT_IDX_DIAG plans or stencils, level by level;
+//  * kTailGrid: every level a stencil with d-linear transfers (the plan code is left out);
+//  * kTailBand: every level a banded plan (variable coefficients).  The row's 3^dim values stay
+//    in registers for the 4 or 5 sweeps of a leg, so a leg reads them once from the caches, and
+//    only for free rows: 729 rows are 93 KB in FP64, which one CU takes in about 2.5 us, as long
+//    as two sweeps; read for each sweep they would bound it.
+enum TailMode { kTailPlan, kTailGrid, kTailBand };
+template<typename DT, int MODE>
 struct TailRow
 {
   uint32_t wd[8];
   DT inv;
   bool masked;
 };
+template<typename DT>
+struct TailRow<DT, kTailBand>
+{
+  uint32_t on;   // bit t: the neighbour of slot t is inside the grid
+  DT inv;
+  bool masked;
+};
 
 // sum of the thread's DIAG-plan row (slot order = CSR order) with x in LDS
 template<typename DT>
-__device__ __forceinline__ DT tail_row_a(const TailRow<DT> R, const int* meta, const DT* tab, uint64_t i, const DT* x)
+__device__ __forceinline__ DT tail_row_a(const TailRow<DT, kTailPlan> R, const int* meta, const DT* tab, uint64_t i, const DT* x)
 {
   const int nt = meta[0];
   DT sum = DT(0);
@@ -3590,14 +3605,102 @@ __device__ __forceinline__ DT tail_row_grid(const DT* sten, TailGeom g, int i, c
   return s;
 }
 
-// the level's row: grid form or plan
-// GRID: every fused level in the grid form (the plan code is left out of the kernel)
-template<bool GRID, typename DT>
-__device__ __forceinline__ DT tail_row(const TailRow<DT>& R, const int* meta, const DT* tab, TailGeom g, uint64_t i,
-                                       const DT* x)
+// a row's values of a banded level: the slots of its neighbours, the rest of v unused
+template<typename DT>
+struct TailBand
 {
-  if constexpr(GRID)
+  DT v[27];
+  DT scale;   // of FP16 values (a power of two; 1 otherwise)
+};
+
+// the slots inside the n1^dim grid, bit t for the offset t of k_band_rows
+__device__ __forceinline__ uint32_t tail_band_on(TailGeom g, int i)
+{
+  const int fx = i % g.n1, fy = (i / g.n1) % g.n1, fz = g.dim == 3 ? i / (g.n1 * g.n1) : 0;
+  uint32_t on = 0;
+#pragma unroll
+  for(int t = 0; t < 27; ++t)
+  {
+    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = g.dim == 3 ? t / 9 - 1 : 0;
+    const bool in = unsigned(fx + dx) < unsigned(g.n1) && unsigned(fy + dy) < unsigned(g.n1) &&
+                    (g.dim == 3 ? unsigned(fz + dz) < unsigned(g.n1) : t < 9);
+    on |= in ? 1u << t : 0u;
+  }
+  return on;
+}
+
+// the stored values of row i (each slot array spans all rows, so every load is in bounds)
+template<typename DT, typename TL>
+__device__ __forceinline__ void tail_band_load(TailBand<DT>& b, const TL& L, uint64_t i)
+{
+  auto take = [&](auto p, auto ns) {
+    using VT = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
+    VT w[decltype(ns)::value];
+#pragma unroll
+    for(int t = 0; t < decltype(ns)::value; ++t) w[t] = p[t * L.n + i];
+#pragma unroll
+    for(int t = 0; t < decltype(ns)::value; ++t) b.v[t] = cvt_val<DT, VT>(w[t]);
+  };
+  auto by_dim = [&](auto p) {
+    if(L.dim == 3)
+      take(p, std::integral_constant<int, 27>());
+    else
+      take(p, std::integral_constant<int, 9>());
+  };
+  if constexpr(std::is_same<DT, float>::value)
+  {
+    b.scale = L.band_f16 ? L.band_scale : DT(1);
+    if(L.band_f16)
+      by_dim(static_cast<const uint16_t*>(L.band));
+    else
+      by_dim(static_cast<const float*>(L.band));
+  }
+  else
+  {
+    b.scale = DT(1);
+    by_dim(L.band);
+  }
+}
+
+// its sum over the neighbours inside the grid in slot order (= CSR order), x in LDS
+template<typename DT>
+__device__ __forceinline__ DT tail_row_band(const TailBand<DT>& b, uint32_t on, TailGeom g, int i, const DT* x)
+{
+  DT s = DT(0);
+  const int m = g.n1, mm = g.n1 * g.n1;
+  auto sum = [&](auto ns) {
+    constexpr int NS = decltype(ns)::value;
+    const bool all = on == (1u << NS) - 1u;
+    if(all)
+    {
+#pragma unroll
+      for(int t = 0; t < NS; ++t)
+        s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
+    }
+    else
+    {
+#pragma unroll
+      for(int t = 0; t < NS; ++t)
+        if(on >> t & 1u)
+          s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
+    }
+  };
+  if(g.dim == 3)
+    sum(std::integral_constant<int, 27>());
+  else
+    sum(std::integral_constant<int, 9>());
+  return std::is_same<DT, float>::value ? s * b.scale : s;   // exact: a power of two
+}
+
+// the level's row
+template<int MODE, typename DT>
+__device__ __forceinline__ DT tail_row(const TailRow<DT, MODE>& R, const TailBand<DT>& band, const int* meta, const DT* tab,
+                                       TailGeom g, uint64_t i, const DT* x)
+{
+  if constexpr(MODE == kTailGrid)
     return tail_row_grid(tab, g, int(i), x);
+  else if constexpr(MODE == kTailBand)
+    return tail_row_band(band, R.on, g, int(i), x);
   else
     return g.dim ? tail_row_grid(tab, g, int(i), x) : tail_row_a(R, meta, tab, i, x);
 }
@@ -3664,9 +3767,9 @@ __device__ __forceinline__ bool tail_skips(double nrm2)
 // Richardson(Jacobi) with `steps` steps from x = 0 on rhs (smooth_impl): with def the last
 // step writes the defect of x_steps into def and x_steps ends in b0; else the last update is
 // accumulated into acc.  b0/b1 are the ping-pong pair.  Thread = row `live ? threadIdx.x : -`.
-template<bool GRID, typename DT>
-__device__ __forceinline__ void tail_smooth(const TailRow<DT> R, bool live, const int* meta, const DT* tab, TailGeom geo,
-                                            int steps, DT omega, bool skip, const DT* rhs, DT* b0, DT* b1, DT* def, DT* acc)
+template<int MODE, typename DT>
+__device__ __forceinline__ void tail_smooth(const TailRow<DT, MODE> R, const TailBand<DT>& band, bool live, const int* meta,
+                                            const DT* tab, TailGeom geo, int steps, DT omega, bool skip, const DT* rhs, DT* b0, DT* b1, DT* def, DT* acc)
 {
   const uint64_t i = threadIdx.x;
   auto B = [&](int k) { return ((steps - k) & 1) ? b1 : b0; };
@@ -3693,7 +3796,7 @@ __device__ __forceinline__ void tail_smooth(const TailRow<DT> R, bool live, cons
     {
       // a filtered row's defect is zero whatever its sum: the sum is skipped
       DT d = DT(0);
-      if(!R.masked) d = dfma(tail_row<GRID>(R, meta, tab, geo, i, xk), DT(-1), rhs[i]);
+      if(!R.masked) d = dfma(tail_row<MODE>(R, band, meta, tab, geo, i, xk), DT(-1), rhs[i]);
       if(mode == 1)
         out[i] = d;
       else
@@ -3720,7 +3823,7 @@ __host__ __device__ inline uint64_t tail_words_bytes(const TT& t)
 }
 
 // TT: feat_mg_tail_t (FP64 cycle) or feat_mg_tail_f32_t (FP32 cycle of the mixed multigrid)
-template<typename DT, typename TT, bool GRID>
+template<typename DT, typename TT, int MODE>
 __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __restrict__ rhs_top,
                                                           const double* __restrict__ nrm_top, DT* __restrict__ sol_top)
 {
@@ -3730,7 +3833,8 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
   const int nl = t.nlevels, c = nl - 1;
   const uint64_t tid = threadIdx.x;
   TailBufs<DT> b[FEAT_MG_TAIL_MAX_LEVELS];
-  TailRow<DT> row[kTailSmoothed];
+  TailRow<DT, MODE> row[kTailSmoothed];
+  TailBand<DT> band;   // the current level's row (kTailBand)
   const int* meta[kTailSmoothed];
   TailGeom geo[kTailSmoothed];
   DT* tabs = lds;   // the smoothed levels' pair-table values, 256 each
@@ -3767,15 +3871,20 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       // grid form: the stencil in the pair table's place, no code words
-      geo[l] = TailGeom{L.sten ? L.dim : 0, int(L.n1)};
-      meta[l] = L.sten ? nullptr : reinterpret_cast<const int*>(L.table + 256) + 256;
-      if(GRID || L.sten)
-        for(int e = threadIdx.x; e < (L.dim == 3 ? 27 : 9); e += kTailThreads) tabs[256 * l + e] = L.sten[e];
-      else
-        for(int e = threadIdx.x; e < 256; e += kTailThreads) tabs[256 * l + e] = L.table[e];
+      geo[l] = TailGeom{MODE == kTailBand || L.sten ? L.dim : 0, int(L.n1)};
+      meta[l] = MODE != kTailPlan || L.sten ? nullptr : reinterpret_cast<const int*>(L.table + 256) + 256;
+      if constexpr(MODE != kTailBand)
+      {
+        if(MODE == kTailGrid || L.sten)
+          for(int e = threadIdx.x; e < (L.dim == 3 ? 27 : 9); e += kTailThreads) tabs[256 * l + e] = L.sten[e];
+        else
+          for(int e = threadIdx.x; e < 256; e += kTailThreads) tabs[256 * l + e] = L.table[e];
+      }
       if(tid < L.n)
       {
-        if(!GRID && !L.sten)
+        if constexpr(MODE == kTailBand)
+          row[l].on = tail_band_on(geo[l], int(tid));
+        else if(MODE == kTailPlan && !L.sten)
         {
           const uint32_t* cw = L.codes + (tid >> 6) * 64 * uint64_t(L.words) + (tid & 63);
 #pragma unroll
@@ -3808,7 +3917,9 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       const bool live = tid < L.n;
-      tail_smooth<GRID>(row[l], live, meta[l], tabs + 256 * l, geo[l], L.pre_steps, L.pre_omega, tail_skips<DT>(nrm[l]),
+      if constexpr(MODE == kTailBand)
+        if(live && !row[l].masked) tail_band_load(band, L, tid);
+      tail_smooth<MODE>(row[l], band, live, meta[l], tabs + 256 * l, geo[l], L.pre_steps, L.pre_omega, tail_skips<DT>(nrm[l]),
                   b[l].rhs, b[l].sol, b[l].tmp, b[l].def, (DT*)nullptr);
       const auto& C = t.lv[l + 1];
       double part = 0.0;
@@ -3818,7 +3929,7 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
         DT v = DT(0);
         if(!is_masked(C.mask, tid))
         {
-          if constexpr(GRID)
+          if constexpr(MODE == kTailGrid)
             v = dfma(tail_rest_grid(TailGeom{L.dim, int(L.n1)}, int(tid), b[l].def), DT(1), DT(0));
           else
             v = dfma(L.dlinear ? tail_rest_grid(TailGeom{L.dim, int(L.n1)}, int(tid), b[l].def)
@@ -3858,12 +3969,14 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       const bool live = tid < L.n;
+      if constexpr(MODE == kTailBand)
+        if(live && !row[l].masked) tail_band_load(band, L, tid);
       if(live)
       {
         DT cc = DT(0);
         if(!row[l].masked)
         {
-          if constexpr(GRID)
+          if constexpr(MODE == kTailGrid)
             cc = dfma(tail_prol_grid(TailGeom{L.dim, int(L.n1)}, int(tid), b[l + 1].sol), DT(1), DT(0));
           else
             cc = dfma(L.dlinear ? tail_prol_grid(TailGeom{L.dim, int(L.n1)}, int(tid), b[l + 1].sol)
@@ -3877,12 +3990,12 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
       if(live)
       {
         DT v = DT(0);
-        if(!row[l].masked) v = dfma(tail_row<GRID>(row[l], meta[l], tabs + 256 * l, geo[l], tid, b[l].sol), DT(-1), b[l].rhs[tid]);
+        if(!row[l].masked) v = dfma(tail_row<MODE>(row[l], band, meta[l], tabs + 256 * l, geo[l], tid, b[l].sol), DT(-1), b[l].rhs[tid]);
         b[l].def[tid] = v;
         part = double(v) * double(v);
       }
       const double dn = tail_sum(part, red);
-      tail_smooth<GRID>(row[l], live, meta[l], tabs + 256 * l, geo[l], L.post_steps, L.post_omega, tail_skips<DT>(dn),
+      tail_smooth<MODE>(row[l], band, live, meta[l], tabs + 256 * l, geo[l], L.post_steps, L.post_omega, tail_skips<DT>(dn),
                   b[l].def, b[l].cor, b[l].tmp, (DT*)nullptr, b[l].sol);
     }
   if(tid < t.lv[0].n) sol_top[tid] = b[0].sol[tid];
@@ -3899,6 +4012,9 @@ int mg_tail_launch(feat_handle_t h, const TT* t, const DT* rhs, const double* rh
       const uint64_t ncn = L.dim == 3 ? nc * nc * nc : nc * nc;
       if((L.sten || L.dlinear) && (L.dim < 2 || L.dim > 3 || n1 < 3 || !(n1 & 1) || nn != L.n || ncn != t->lv[l + 1].n))
         return fail(FEAT_ERR_INVALID, "fused coarse levels: grid form inconsistent with the level sizes");
+      if(L.band && (L.dim < 2 || L.dim > 3 || n1 < 3 || n1 > uint64_t(kTailThreads) || nn != L.n))
+        return fail(FEAT_ERR_INVALID, "fused coarse levels: banded form inconsistent with the level sizes");
+      if(!L.band != !t->lv[0].band) return fail(FEAT_ERR_INVALID, "fused coarse levels: banded and other levels mixed");
     }
   if(!h || !t || !rhs || !rhs_nrm2 || !sol || t->nlevels < 2 || t->nlevels > FEAT_MG_TAIL_MAX_LEVELS ||
      !t->coarse_inverse)
@@ -3910,7 +4026,7 @@ int mg_tail_launch(feat_handle_t h, const TT* t, const DT* rhs, const double* rh
     words += (l + 1 < t->nlevels ? 5 * L.n + 256 : 2 * L.n);
     if(L.n > uint64_t(kTailThreads)) return fail(FEAT_ERR_INVALID, "fused coarse levels: a level has more than 1024 rows");
     if(l + 1 < t->nlevels &&
-       (!L.table || !L.codes || L.words > 8 || !L.inv_diag || !L.r_val || !L.r_col || !L.r_ptr || !L.p_val ||
+       ((!L.band && (!L.table || !L.codes || L.words > 8)) || !L.inv_diag || !L.r_val || !L.r_col || !L.r_ptr || !L.p_val ||
         !L.p_col || !L.p_ptr || L.pre_steps < 1 || L.post_steps < 1))
       return fail(FEAT_ERR_INVALID, "fused coarse levels: incomplete level");
   }
@@ -3922,10 +4038,12 @@ int mg_tail_launch(feat_handle_t h, const TT* t, const DT* rhs, const double* rh
   // every smoothed level in the grid form: the kernel without the plan code
   bool grid = true;
   for(int l = 0; l + 1 < t->nlevels; ++l) grid = grid && t->lv[l].sten && t->lv[l].dlinear;
-  if(grid)
-    hipLaunchKernelGGL((k_mg_tail<DT, TT, true>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
+  if(t->lv[0].band)
+    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailBand>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
+  else if(grid)
+    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailGrid>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
   else
-    hipLaunchKernelGGL((k_mg_tail<DT, TT, false>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
+    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailPlan>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
   return check_launch(name);
 }
 

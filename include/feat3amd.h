@@ -910,7 +910,7 @@ int feat_ilu_done_symbolic(feat_ilu_t s);
  * value is computed with the same operations in the same order as the separate launches
  * (matrix sums in CSR / slot order), so the solution is bit-identical; the |.|^2 sums
  * feeding the smoothers' skip rule (exact zero or non-finite) are summed in another order.
- * lv[0 .. nlevels-2]: smoothed levels (A as a FEAT_IDX_DIAG plan, restriction to and
+ * lv[0 .. nlevels-2]: smoothed levels (A as a FEAT_IDX_DIAG or a banded plan, restriction to and
  * prolongation from the next level as CSR); lv[nlevels-1]: the coarsest level (n, mask).
  * rhs / rhs_nrm2: level t's right-hand side and |rhs|^2 (device); sol: level t's solution
  * (written).  The caller keeps 8 bytes x (5 n + 256 over the smoothed levels + 2 n coarse)
@@ -938,6 +938,10 @@ typedef struct {
   uint32_t n1;
   const double* sten;
   int dlinear;
+  /* banded form (NULL: unused; then on no smoothed level): the values of the level's
+   * FEAT_FMT_BANDED plan, read instead of a dictionary plan (table and codes may be NULL);
+   * dim and n1 are set with it. */
+  const double* band;
 } feat_mg_tail_level_t;
 typedef struct {
   int nlevels;
@@ -964,6 +968,9 @@ typedef struct {
   uint32_t n1;
   const float* sten;
   int dlinear;
+  const void* band;            /* banded form: FP32 values, or with band_f16 FP16 values, */
+  int band_f16;                /* whose row sums are multiplied by band_scale (the plan's */
+  float band_scale;            /* scale, a power of two) */
 } feat_mg_tail_level_f32_t;
 typedef struct {
   int nlevels;

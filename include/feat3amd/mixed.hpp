@@ -115,9 +115,9 @@ namespace feat3amd
 
       /// The coarse levels that run as one LDS-resident workgroup (feat_mg_tail_f32): the
       /// longest run ending at the coarsest level, starting at level 1 or below, whose
-      /// vectors fit the LDS budget, with FP32 diagonal-dictionary plans, FP32-valued transfer
-      /// plans (an FP16-valued cycle uses FP32 plans where the matrix has a dictionary plan)
-      /// and a direct coarse solve.
+      /// vectors fit the LDS budget, with FP32 diagonal-dictionary plans (or, all of them,
+      /// banded plans), FP32-valued transfer plans (an FP16-valued cycle uses FP32 plans where
+      /// the matrix has a dictionary plan) or d-linear transfers, and a direct coarse solve.
       void _build_tail()
       {
         _tail_built = true;
@@ -131,10 +131,13 @@ namespace feat3amd
         {
           const auto& l = _h->levels[s];
           const feat_matrix_f32_t& A = plan(*l.matrix);
-          const bool f16 = plan(l.transfer->get_mat_rest()).value_kind == FEAT_VAL_F16 ||
-                           plan(l.transfer->get_mat_prol()).value_kind == FEAT_VAL_F16;
+          const bool band = A.format == FEAT_FMT_BANDED;
+          const bool dlin = s < _grid.size() && _grid[s].dlinear;
+          const bool f16 = !dlin && (plan(l.transfer->get_mat_rest()).value_kind == FEAT_VAL_F16 ||
+                                     plan(l.transfer->get_mat_prol()).value_kind == FEAT_VAL_F16);
           const uint64_t need = words + 5 * l.matrix->rows() + 256;   // vectors and the pair table
-          if(f16 || A.index != FEAT_IDX_DIAG || A.slice_words > 8 || need * sizeof(float) > FEAT_MG_TAIL_MAX_LDS ||
+          if(f16 || (!band && (A.index != FEAT_IDX_DIAG || A.slice_words > 8)) ||
+             band != (plan(*_h->levels[c - 1].matrix).format == FEAT_FMT_BANDED) || need * sizeof(float) > FEAT_MG_TAIL_MAX_LDS ||
              c - s + 1 > FEAT_MG_TAIL_MAX_LEVELS || l.matrix->rows() > FEAT_MG_TAIL_MAX_ROWS)
             break;
           words = need;
@@ -151,9 +154,20 @@ namespace feat3amd
           d.mask = lv.filter->mask();
           if(s == c) break;
           const feat_matrix_f32_t& A = plan(*lv.matrix);
-          d.table = static_cast<const float*>(A.val);
-          d.codes = static_cast<const uint32_t*>(A.col);
-          d.words = A.slice_words;
+          if(A.format == FEAT_FMT_BANDED)
+          {
+            d.band = A.val;
+            d.band_f16 = A.value_kind == FEAT_VAL_F16 ? 1 : 0;
+            d.band_scale = float(A.scale);
+            d.n1 = A.slice_words;
+            d.dim = uint64_t(d.n1) * d.n1 == d.n ? 2 : 3;
+          }
+          else
+          {
+            d.table = static_cast<const float*>(A.val);
+            d.codes = static_cast<const uint32_t*>(A.col);
+            d.words = A.slice_words;
+          }
           // one inverted diagonal serves both smoothers: their FP64 sources must be one vector
           auto* pre = static_cast<RichType*>(lv.pre.get());
           auto* post = static_cast<RichType*>(lv.post.get());
@@ -177,7 +191,7 @@ namespace feat3amd
             d.dim = _grid[s].dim;
             d.n1 = _grid[s].n1;
             d.dlinear = _grid[s].dlinear ? 1 : 0;
-            d.sten = _grid_sten[s].size() ? _grid_sten[s].get() : nullptr;
+            d.sten = _grid_sten[s].size() && !d.band ? _grid_sten[s].get() : nullptr;
           }
         }
         _tail.coarse_inverse = static_cast<DirectType*>(_h->levels[c].coarse.get())->inverse();

@@ -709,7 +709,8 @@ namespace feat3amd
 
       /// The coarse levels that run as one LDS-resident workgroup (feat_mg_tail_f64): the
       /// longest run ending at the coarsest level, starting at level 1 or below, whose
-      /// vectors fit the LDS budget, with diagonal-dictionary plans and a direct coarse solve.
+      /// vectors fit the LDS budget, with diagonal-dictionary plans (or, all of them, banded
+      /// plans) and a direct coarse solve.
       void _build_tail()
       {
         _tail_built = true;
@@ -725,7 +726,9 @@ namespace feat3amd
           const auto& l = _h->levels[s];
           const feat_matrix_f64_t& A = l.matrix->exec();
           const uint64_t need = doubles + 5 * l.matrix->rows() + 256;   // vectors and the pair table
-          if(A.index != FEAT_IDX_DIAG || A.slice_words > 8 || need * sizeof(double) > FEAT_MG_TAIL_MAX_LDS ||
+          const bool band = A.format == FEAT_FMT_BANDED;
+          if((!band && (A.index != FEAT_IDX_DIAG || A.slice_words > 8)) ||
+             band != (_h->levels[c - 1].matrix->exec().format == FEAT_FMT_BANDED) || need * sizeof(double) > FEAT_MG_TAIL_MAX_LDS ||
              c - s + 1 > FEAT_MG_TAIL_MAX_LEVELS || l.matrix->rows() > FEAT_MG_TAIL_MAX_ROWS)
             break;
           doubles = need;
@@ -742,9 +745,18 @@ namespace feat3amd
           d.mask = l.filter->mask();
           if(s == c) break;
           const feat_matrix_f64_t& A = l.matrix->exec();
-          d.table = static_cast<const double*>(A.val);
-          d.codes = static_cast<const uint32_t*>(A.col);
-          d.words = A.slice_words;
+          if(A.format == FEAT_FMT_BANDED)
+          {
+            d.band = A.val;
+            d.n1 = A.slice_words;
+            d.dim = uint64_t(d.n1) * d.n1 == d.n ? 2 : 3;
+          }
+          else
+          {
+            d.table = static_cast<const double*>(A.val);
+            d.codes = static_cast<const uint32_t*>(A.col);
+            d.words = A.slice_words;
+          }
           auto* pre = static_cast<RichType*>(l.pre.get());
           auto* post = static_cast<RichType*>(l.post.get());
           d.inv_diag = (const double*)pre->fusable_jacobi()->inv_diag().elements();
@@ -767,7 +779,7 @@ namespace feat3amd
             d.dim = _grid[s].dim;
             d.n1 = _grid[s].n1;
             d.dlinear = _grid[s].dlinear ? 1 : 0;
-            d.sten = _grid_sten[s].size() ? _grid_sten[s].get() : nullptr;
+            d.sten = _grid_sten[s].size() && !d.band ? _grid_sten[s].get() : nullptr;
           }
         }
         _tail.coarse_inverse = static_cast<DirectCoarseSolver<Matrix_, Filter_>*>(_h->levels[c].coarse.get())->inverse();
