@@ -3546,25 +3546,24 @@ constexpr int kTailSmoothed = FEAT_MG_TAIL_MAX_LEVELS - 1;
 // MODE: how the smoothed levels hold their rows (one form for all of them).
 //  * kTailPlan: FEAT_IDX_DIAG plans or stencils, level by level;
 //  * kTailGrid: every level a stencil with d-linear transfers (the plan code is left out);
-//  * kTailBand: every level a banded plan (variable coefficients).  The row's 3^dim values stay
-//    in registers for the 4 or 5 sweeps of a leg, so a leg reads them once from the caches, and
-//    only for free rows: 729 rows are 93 KB in FP64, which one CU takes in about 2.5 us, as long
-//    as two sweeps; read for each sweep they would bound it.
-enum TailMode { kTailPlan, kTailGrid, kTailBand };
+//  * kTailBand2, kTailBand3: every level a banded plan (variable coefficients) in 2D or 3D.  The
+//    row's 3^dim values stay in registers for the 4 or 5 sweeps of a leg, so a leg reads them
+//    once from the caches, and only for free rows; a kernel per dimension keeps them out of
+//    scratch (with the dimension at run time a third of them went there: 63 us instead of 37).
+//    729 + 125 rows over a direct 27, V(4,4): 37 us in FP64, 32 us in FP32 with FP16 values,
+//    against about 110 us of 25 launches.
+enum TailMode { kTailPlan, kTailGrid, kTailBand2, kTailBand3 };
 template<typename DT, int MODE>
 struct TailRow
 {
   uint32_t wd[8];
+  uint32_t on;   // banded: bit t: the neighbour of slot t is inside the grid
   DT inv;
   bool masked;
 };
-template<typename DT>
-struct TailRow<DT, kTailBand>
-{
-  uint32_t on;   // bit t: the neighbour of slot t is inside the grid
-  DT inv;
-  bool masked;
-};
+// slots of a banded row (1: the other forms have none)
+constexpr int tail_slots(int mode) { return mode == kTailBand3 ? 27 : mode == kTailBand2 ? 9 : 1; }
+constexpr bool tail_banded(int mode) { return mode >= kTailBand2; }
 
 // sum of the thread's DIAG-plan row (slot order = CSR order) with x in LDS
 template<typename DT>
@@ -3605,101 +3604,87 @@ __device__ __forceinline__ DT tail_row_grid(const DT* sten, TailGeom g, int i, c
   return s;
 }
 
-// a row's values of a banded level: the slots of its neighbours, the rest of v unused
-template<typename DT>
+// a row's values of a banded level
+template<typename DT, int NS>
 struct TailBand
 {
-  DT v[27];
+  DT v[NS];
   DT scale;   // of FP16 values (a power of two; 1 otherwise)
 };
 
 // the slots inside the n1^dim grid, bit t for the offset t of k_band_rows
+template<int NS>
 __device__ __forceinline__ uint32_t tail_band_on(TailGeom g, int i)
 {
-  const int fx = i % g.n1, fy = (i / g.n1) % g.n1, fz = g.dim == 3 ? i / (g.n1 * g.n1) : 0;
+  const int fx = i % g.n1, fy = NS == 27 ? (i / g.n1) % g.n1 : i / g.n1, fz = NS == 27 ? i / (g.n1 * g.n1) : 0;
   uint32_t on = 0;
 #pragma unroll
-  for(int t = 0; t < 27; ++t)
+  for(int t = 0; t < NS; ++t)
   {
-    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = g.dim == 3 ? t / 9 - 1 : 0;
+    const int dx = t % 3 - 1, dy = (t / 3) % 3 - 1, dz = NS == 27 ? t / 9 - 1 : 0;
     const bool in = unsigned(fx + dx) < unsigned(g.n1) && unsigned(fy + dy) < unsigned(g.n1) &&
-                    (g.dim == 3 ? unsigned(fz + dz) < unsigned(g.n1) : t < 9);
+                    unsigned(fz + dz) < unsigned(g.n1);
     on |= in ? 1u << t : 0u;
   }
   return on;
 }
 
 // the stored values of row i (each slot array spans all rows, so every load is in bounds)
-template<typename DT, typename TL>
-__device__ __forceinline__ void tail_band_load(TailBand<DT>& b, const TL& L, uint64_t i)
+template<typename DT, int NS, typename VT>
+__device__ __forceinline__ void tail_band_take(TailBand<DT, NS>& b, const VT* p, uint64_t n, uint32_t i)
 {
-  auto take = [&](auto p, auto ns) {
-    using VT = std::remove_const_t<std::remove_pointer_t<decltype(p)>>;
-    VT w[decltype(ns)::value];
+  VT w[NS];
 #pragma unroll
-    for(int t = 0; t < decltype(ns)::value; ++t) w[t] = p[t * L.n + i];
+  for(int t = 0; t < NS; ++t) w[t] = (p + t * n)[i];
 #pragma unroll
-    for(int t = 0; t < decltype(ns)::value; ++t) b.v[t] = cvt_val<DT, VT>(w[t]);
-  };
-  auto by_dim = [&](auto p) {
-    if(L.dim == 3)
-      take(p, std::integral_constant<int, 27>());
-    else
-      take(p, std::integral_constant<int, 9>());
-  };
+  for(int t = 0; t < NS; ++t) b.v[t] = cvt_val<DT, VT>(w[t]);
+}
+template<typename DT, int NS, typename TL>
+__device__ __forceinline__ void tail_band_load(TailBand<DT, NS>& b, const TL& L, uint32_t i)
+{
   if constexpr(std::is_same<DT, float>::value)
   {
-    b.scale = L.band_f16 ? L.band_scale : DT(1);
     if(L.band_f16)
-      by_dim(static_cast<const uint16_t*>(L.band));
+      tail_band_take(b, static_cast<const uint16_t*>(L.band), L.n, i);
     else
-      by_dim(static_cast<const float*>(L.band));
+      tail_band_take(b, static_cast<const float*>(L.band), L.n, i);
+    b.scale = L.band_f16 ? L.band_scale : DT(1);
   }
   else
-  {
-    b.scale = DT(1);
-    by_dim(L.band);
-  }
+    tail_band_take(b, L.band, L.n, i);
 }
 
 // its sum over the neighbours inside the grid in slot order (= CSR order), x in LDS
-template<typename DT>
-__device__ __forceinline__ DT tail_row_band(const TailBand<DT>& b, uint32_t on, TailGeom g, int i, const DT* x)
+template<typename DT, int NS>
+__device__ __forceinline__ DT tail_row_band(const TailBand<DT, NS>& b, uint32_t on, TailGeom g, int i, const DT* x)
 {
   DT s = DT(0);
-  const int m = g.n1, mm = g.n1 * g.n1;
-  auto sum = [&](auto ns) {
-    constexpr int NS = decltype(ns)::value;
-    const bool all = on == (1u << NS) - 1u;
-    if(all)
-    {
+  const int m = g.n1, mm = NS == 27 ? g.n1 * g.n1 : 0;
+  if(on == (1u << NS) - 1u)
+  {
 #pragma unroll
-      for(int t = 0; t < NS; ++t)
-        s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
-    }
-    else
-    {
-#pragma unroll
-      for(int t = 0; t < NS; ++t)
-        if(on >> t & 1u)
-          s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
-    }
-  };
-  if(g.dim == 3)
-    sum(std::integral_constant<int, 27>());
+    for(int t = 0; t < NS; ++t)
+      s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
+  }
   else
-    sum(std::integral_constant<int, 9>());
-  return std::is_same<DT, float>::value ? s * b.scale : s;   // exact: a power of two
+  {
+#pragma unroll
+    for(int t = 0; t < NS; ++t)
+      if(on >> t & 1u)
+        s = dfma(b.v[t], x[i + (t % 3 - 1) + ((t / 3) % 3 - 1) * m + (NS == 27 ? t / 9 - 1 : 0) * mm], s);
+  }
+  if constexpr(std::is_same<DT, float>::value) s = s * b.scale;   // exact: a power of two
+  return s;
 }
 
 // the level's row
 template<int MODE, typename DT>
-__device__ __forceinline__ DT tail_row(const TailRow<DT, MODE>& R, const TailBand<DT>& band, const int* meta, const DT* tab,
-                                       TailGeom g, uint64_t i, const DT* x)
+__device__ __forceinline__ DT tail_row(const TailRow<DT, MODE>& R, const TailBand<DT, tail_slots(MODE)>& band,
+                                       const int* meta, const DT* tab, TailGeom g, uint64_t i, const DT* x)
 {
   if constexpr(MODE == kTailGrid)
     return tail_row_grid(tab, g, int(i), x);
-  else if constexpr(MODE == kTailBand)
+  else if constexpr(tail_banded(MODE))
     return tail_row_band(band, R.on, g, int(i), x);
   else
     return g.dim ? tail_row_grid(tab, g, int(i), x) : tail_row_a(R, meta, tab, i, x);
@@ -3768,8 +3753,8 @@ __device__ __forceinline__ bool tail_skips(double nrm2)
 // step writes the defect of x_steps into def and x_steps ends in b0; else the last update is
 // accumulated into acc.  b0/b1 are the ping-pong pair.  Thread = row `live ? threadIdx.x : -`.
 template<int MODE, typename DT>
-__device__ __forceinline__ void tail_smooth(const TailRow<DT, MODE> R, const TailBand<DT>& band, bool live, const int* meta,
-                                            const DT* tab, TailGeom geo, int steps, DT omega, bool skip, const DT* rhs, DT* b0, DT* b1, DT* def, DT* acc)
+__device__ __forceinline__ void tail_smooth(const TailRow<DT, MODE> R, const TailBand<DT, tail_slots(MODE)>& band, bool live,
+                                            const int* meta, const DT* tab, TailGeom geo, int steps, DT omega, bool skip, const DT* rhs, DT* b0, DT* b1, DT* def, DT* acc)
 {
   const uint64_t i = threadIdx.x;
   auto B = [&](int k) { return ((steps - k) & 1) ? b1 : b0; };
@@ -3834,7 +3819,7 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
   const uint64_t tid = threadIdx.x;
   TailBufs<DT> b[FEAT_MG_TAIL_MAX_LEVELS];
   TailRow<DT, MODE> row[kTailSmoothed];
-  TailBand<DT> band;   // the current level's row (kTailBand)
+  TailBand<DT, tail_slots(MODE)> band;   // the current level's row
   const int* meta[kTailSmoothed];
   TailGeom geo[kTailSmoothed];
   DT* tabs = lds;   // the smoothed levels' pair-table values, 256 each
@@ -3871,9 +3856,9 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       // grid form: the stencil in the pair table's place, no code words
-      geo[l] = TailGeom{MODE == kTailBand || L.sten ? L.dim : 0, int(L.n1)};
+      geo[l] = TailGeom{tail_banded(MODE) || L.sten ? L.dim : 0, int(L.n1)};
       meta[l] = MODE != kTailPlan || L.sten ? nullptr : reinterpret_cast<const int*>(L.table + 256) + 256;
-      if constexpr(MODE != kTailBand)
+      if constexpr(!tail_banded(MODE))
       {
         if(MODE == kTailGrid || L.sten)
           for(int e = threadIdx.x; e < (L.dim == 3 ? 27 : 9); e += kTailThreads) tabs[256 * l + e] = L.sten[e];
@@ -3882,8 +3867,8 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
       }
       if(tid < L.n)
       {
-        if constexpr(MODE == kTailBand)
-          row[l].on = tail_band_on(geo[l], int(tid));
+        if constexpr(tail_banded(MODE))
+          row[l].on = tail_band_on<tail_slots(MODE)>(geo[l], int(tid));
         else if(MODE == kTailPlan && !L.sten)
         {
           const uint32_t* cw = L.codes + (tid >> 6) * 64 * uint64_t(L.words) + (tid & 63);
@@ -3917,8 +3902,8 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       const bool live = tid < L.n;
-      if constexpr(MODE == kTailBand)
-        if(live && !row[l].masked) tail_band_load(band, L, tid);
+      if constexpr(tail_banded(MODE))
+        if(live && !row[l].masked) tail_band_load(band, L, threadIdx.x);
       tail_smooth<MODE>(row[l], band, live, meta[l], tabs + 256 * l, geo[l], L.pre_steps, L.pre_omega, tail_skips<DT>(nrm[l]),
                   b[l].rhs, b[l].sol, b[l].tmp, b[l].def, (DT*)nullptr);
       const auto& C = t.lv[l + 1];
@@ -3969,8 +3954,8 @@ __global__ __launch_bounds__(kTailThreads) void k_mg_tail(TT t, const DT* __rest
     {
       const auto& L = t.lv[l];
       const bool live = tid < L.n;
-      if constexpr(MODE == kTailBand)
-        if(live && !row[l].masked) tail_band_load(band, L, tid);
+      if constexpr(tail_banded(MODE))
+        if(live && !row[l].masked) tail_band_load(band, L, threadIdx.x);
       if(live)
       {
         DT cc = DT(0);
@@ -4014,7 +3999,8 @@ int mg_tail_launch(feat_handle_t h, const TT* t, const DT* rhs, const double* rh
         return fail(FEAT_ERR_INVALID, "fused coarse levels: grid form inconsistent with the level sizes");
       if(L.band && (L.dim < 2 || L.dim > 3 || n1 < 3 || n1 > uint64_t(kTailThreads) || nn != L.n))
         return fail(FEAT_ERR_INVALID, "fused coarse levels: banded form inconsistent with the level sizes");
-      if(!L.band != !t->lv[0].band) return fail(FEAT_ERR_INVALID, "fused coarse levels: banded and other levels mixed");
+      if(!L.band != !t->lv[0].band || (L.band && L.dim != t->lv[0].dim))
+        return fail(FEAT_ERR_INVALID, "fused coarse levels: banded and other levels mixed");
     }
   if(!h || !t || !rhs || !rhs_nrm2 || !sol || t->nlevels < 2 || t->nlevels > FEAT_MG_TAIL_MAX_LEVELS ||
      !t->coarse_inverse)
@@ -4038,8 +4024,10 @@ int mg_tail_launch(feat_handle_t h, const TT* t, const DT* rhs, const double* rh
   // every smoothed level in the grid form: the kernel without the plan code
   bool grid = true;
   for(int l = 0; l + 1 < t->nlevels; ++l) grid = grid && t->lv[l].sten && t->lv[l].dlinear;
-  if(t->lv[0].band)
-    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailBand>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
+  if(t->lv[0].band && t->lv[0].dim == 2)
+    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailBand2>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
+  else if(t->lv[0].band)
+    hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailBand3>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
   else if(grid)
     hipLaunchKernelGGL((k_mg_tail<DT, TT, kTailGrid>), dim3(1), dim3(kTailThreads), lds, h->stream, *t, rhs, rhs_nrm2, sol);
   else
