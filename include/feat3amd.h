@@ -912,7 +912,7 @@ int feat_ilu_done_symbolic(feat_ilu_t s);
  * feeding the smoothers' skip rule (exact zero or non-finite) are summed in another order.
  * lv[0 .. nlevels-2]: smoothed levels (A as a FEAT_IDX_DIAG or a banded plan, restriction to and
  * prolongation from the next level as CSR); lv[nlevels-1]: the coarsest level (n, mask).
- * rhs / rhs_nrm2: level t's right-hand side and |rhs|^2 (device); sol: level t's solution
+ * rhs / rhs_nrm2: level t's right-hand side and |rhs|^2 (device; unused with sum_rhs); sol: level t's solution
  * (written).  The caller keeps 8 bytes x (5 n + 256 over the smoothed levels + 2 n coarse)
  * within FEAT_MG_TAIL_MAX_LDS bytes (when the coarse inverse, 8 n_c^2 bytes, also fits, it
  * is staged in LDS).  No counterpart in the reference (a launch-count fusion). */
@@ -947,6 +947,7 @@ typedef struct {
   int nlevels;
   feat_mg_tail_level_t lv[FEAT_MG_TAIL_MAX_LEVELS];
   const double* coarse_inverse;   /* n x n row-major inverse of the filtered coarsest matrix */
+  int sum_rhs;                    /* 1: |rhs|^2 is summed in the kernel, rhs_nrm2 may be NULL */
 } feat_mg_tail_t;
 int feat_mg_tail_f64(feat_handle_t h, const feat_mg_tail_t* t, const double* rhs, const double* rhs_nrm2, double* sol);
 /* The same for the FP32 V-cycle of the mixed-precision multigrid (feat_rj_smooth_f32,
@@ -976,6 +977,7 @@ typedef struct {
   int nlevels;
   feat_mg_tail_level_f32_t lv[FEAT_MG_TAIL_MAX_LEVELS];
   const double* coarse_inverse;
+  int sum_rhs;
 } feat_mg_tail_f32_t;
 int feat_mg_tail_f32(feat_handle_t h, const feat_mg_tail_f32_t* t, const float* rhs, const double* rhs_nrm2, float* sol);
 

@@ -146,6 +146,7 @@ namespace feat3amd
         if(t == c) return;
         _tail = feat_mg_tail_f32_t{};
         _tail.nlevels = int(c - t + 1);
+        _tail.sum_rhs = 1;
         for(Index s = t; s <= c; ++s)
         {
           auto& lv = _h->levels[s];
@@ -330,11 +331,11 @@ namespace feat3amd
                 "FP32 pre-smoothing");
           const feat_matrix_f32_t& R = _rest(i);
           check(feat_apply_masked_f32(hd, &R, _l[i + 1].rhs.elements(), l.def.elements(), _h->levels[i + 1].filter->mask(),
-                                      _fw.scalar(2 + i + 1), ws),
+                                      _tail_t && i + 1 == t ? nullptr : _fw.scalar(2 + i + 1), ws),
                 "FP32 restriction");
         }
         if(_tail_t)
-          check(feat_mg_tail_f32(hd, &_tail, _l[t].rhs.elements(), nrm_of(t), _l[t].sol.elements()),
+          check(feat_mg_tail_f32(hd, &_tail, _l[t].rhs.elements(), nullptr, _l[t].sol.elements()),
                 "FP32 fused coarse levels");
         else
         {

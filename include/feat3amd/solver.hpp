@@ -737,6 +737,7 @@ namespace feat3amd
         if(t == c) return;
         _tail = feat_mg_tail_t{};
         _tail.nlevels = int(c - t + 1);
+        _tail.sum_rhs = 1;
         for(Index s = t; s <= c; ++s)
         {
           auto& l = _h->levels[s];
@@ -954,6 +955,9 @@ namespace feat3amd
           return i == 0 ? (double*)cor.elements() : (double*)_h->levels[i].sol.elements();
         };
         auto nrm_of = [&](Index i) -> const double* { return i == 0 ? def_nrm2 : _fw.scalar(2 + i); };
+        // the fused coarse levels sum the |rhs|^2 that their first smoother's skip rule needs
+        // themselves: a restriction without a grid reduction
+        auto rest_nrm = [&](Index i) -> double* { return _tail_t && i == t ? nullptr : _fw.scalar(2 + i); };
         // restriction leg (multigrid.hpp:1713-1840)
         bool x1_ready = top_x1;
         for(Index i = 0; i < t; ++i)
@@ -975,19 +979,19 @@ namespace feat3amd
           {
             auto* pc = static_cast<RichType*>(lc.pre.get());
             check(feat_apply_masked_first_f64(hd, &R, (double*)lc.rhs.elements(), (const double*)l.def.elements(),
-                                              lc.filter->mask(), _fw.scalar(2 + i + 1),
+                                              lc.filter->mask(), rest_nrm(i + 1),
                                               (const double*)pc->fusable_jacobi()->inv_diag().elements(), pc->omega(),
                                               x1, ws),
                   "MultiGrid restriction");
           }
           else
             check(feat_apply_masked_f64(hd, &R, (double*)lc.rhs.elements(), (const double*)l.def.elements(),
-                                        lc.filter->mask(), _fw.scalar(2 + i + 1), nullptr, nullptr, ws),
+                                        lc.filter->mask(), rest_nrm(i + 1), nullptr, nullptr, ws),
                   "MultiGrid restriction");
           x1_ready = x1 != nullptr;
         }
         if(_tail_t)
-          check(feat_mg_tail_f64(hd, &_tail, rhs_of(t), nrm_of(t), sol_of(t)), "MultiGrid fused coarse levels");
+          check(feat_mg_tail_f64(hd, &_tail, rhs_of(t), nullptr, sol_of(t)), "MultiGrid fused coarse levels");
         // coarse solve (multigrid.hpp:1526-1589)
         else
         {
