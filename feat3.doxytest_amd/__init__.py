@@ -189,6 +189,13 @@ KERNEL_API = [
     ("feat_prol_add_f32", _i, [_vp, C.POINTER(Matrix), _vp, _vp, _vp]),
     ("feat_rj_smooth_f32", _i, [_vp, C.POINTER(Matrix), _vp, _vp, _i, _f, _vp, _vp, _vp, _vp, _vp, _vp,
                                 C.POINTER(ReduceWs)]),
+    ("feat_convert_first_f64_f32", _i, [_vp, _vp, _vp, _u64, _vp, _vp, _f, _vp]),
+    ("feat_apply_masked_first_f32", _i, [_vp, C.POINTER(Matrix), _vp, _vp, _vp, _vp, _vp, _f, _vp,
+                                         C.POINTER(ReduceWs)]),
+    ("feat_defect_first_f32", _i, [_vp, C.POINTER(Matrix), _vp, _vp, _vp, _vp, _vp, _vp, _f, _vp,
+                                   C.POINTER(ReduceWs)]),
+    ("feat_rj_smooth_from1_f32", _i, [_vp, C.POINTER(Matrix), _vp, _vp, _i, _f, _vp, _vp, _vp, _vp, _vp, _vp,
+                                      C.POINTER(ReduceWs)]),
     ("feat_dense_gemv_f32", _i, [_vp, _i, _vp, _vp, _vp, _vp]),
     ("feat_convert_dot_f32_f64", _i, [_vp, _vp, _vp, _vp, _u64, _vp, C.POINTER(ReduceWs)]),
     ("feat_dense_gemv_mixed", _i, [_vp, _i, _vp, _vp, _vp, _vp]),

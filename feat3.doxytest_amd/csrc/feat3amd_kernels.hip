@@ -1956,6 +1956,18 @@ __global__ void k_smooth_first(DT* x1, const DT* inv, const DT* rhs, const uint3
   grid_reduce_finish(gr, 0.0, a1);
 }
 
+// o = in in FP32, with the first iterate of the smoother that takes o as its right-hand side
+__global__ __launch_bounds__(kThreads) void k_convert_first(float* o, const double* in, uint64_t n, FirstIter<float> first,
+                                                            const uint32_t* mask)
+{
+  for(uint64_t i = blockIdx.x * uint64_t(blockDim.x) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * blockDim.x)
+  {
+    const float v = float(in[i]);
+    o[i] = v;
+    first.store(i, v, first.inv[i], is_masked(mask, i));
+  }
+}
+
 template<typename DT>
 __global__ void k_dense_gemv(int n, const DT* ainv, const DT* b, DT* x, const uint32_t* mask)
 {
@@ -3509,6 +3521,42 @@ int feat_rj_smooth_f32(feat_handle_t h, const feat_matrix_f32_t* A, const float*
 {
   return smooth_impl<float>(h, A, inv_diag, mask, steps, omega, rhs, rhs_nrm2, x, tmp, d_out, acc, nullptr, nullptr,
                             ws, "feat_rj_smooth_f32");
+}
+
+// the FP32 producers of a smoother's first iterate (FP64: feat_defect_first_f64 and so on)
+int feat_convert_first_f64_f32(feat_handle_t h, float* o, const double* in, uint64_t n, const float* inv_diag,
+                               const uint32_t* mask, float omega, float* x1)
+{
+  if(!h || (n && (!o || !in || !inv_diag || !x1))) return fail(FEAT_ERR_INVALID, "feat_convert_first_f64_f32: null argument");
+  if(x1 == o && n) return fail(FEAT_ERR_ALIAS, "feat_convert_first_f64_f32: x1 aliases the output");
+  if(!n) return FEAT_OK;
+  hipLaunchKernelGGL(k_convert_first, dim3(grid_for(n, 4)), dim3(kThreads), 0, h->stream, o, in, n,
+                     FirstIter<float>{inv_diag, x1, omega}, mask);
+  return check_launch("feat_convert_first_f64_f32");
+}
+
+int feat_apply_masked_first_f32(feat_handle_t h, const feat_matrix_f32_t* A, float* r, const float* x, const uint32_t* mask,
+                                double* nrm2, const float* inv_diag, float omega, float* x1, const feat_reduce_ws_t* ws)
+{
+  if(!x1) return fail(FEAT_ERR_INVALID, "feat_apply_masked_first_f32: null x1");
+  return masked_impl<float>(h, A, r, x, mask, nrm2, (const float*)nullptr, nullptr, ws, "feat_apply_masked_first_f32",
+                            FirstIter<float>{inv_diag, x1, omega});
+}
+
+int feat_defect_first_f32(feat_handle_t h, const feat_matrix_f32_t* A, float* d, const float* rhs, const float* x,
+                          const uint32_t* mask, double* nrm2, const float* inv_diag, float omega, float* x1,
+                          const feat_reduce_ws_t* ws)
+{
+  if(!x1) return fail(FEAT_ERR_INVALID, "feat_defect_first_f32: null x1");
+  return defect_impl<float>(h, A, d, rhs, x, mask, nrm2, ws, "feat_defect_first_f32", FirstIter<float>{inv_diag, x1, omega});
+}
+
+int feat_rj_smooth_from1_f32(feat_handle_t h, const feat_matrix_f32_t* A, const float* inv_diag, const uint32_t* mask,
+                             int steps, float omega, const float* rhs, const double* rhs_nrm2, float* x, float* tmp,
+                             float* d_out, float* acc, const feat_reduce_ws_t* ws)
+{
+  return smooth_impl<float>(h, A, inv_diag, mask, steps, omega, rhs, rhs_nrm2, x, tmp, d_out, acc, nullptr, nullptr, ws,
+                            "feat_rj_smooth_from1_f32", true);
 }
 
 int feat_dense_gemv_f32(feat_handle_t h, int n, const float* ainv, const float* b, float* x, const uint32_t* mask)

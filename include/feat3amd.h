@@ -446,6 +446,21 @@ int feat_rj_smooth_f32(feat_handle_t h, const feat_matrix_f32_t* A, const float*
                        const uint32_t* mask, int steps, float omega, const float* rhs,
                        const double* rhs_nrm2, float* x, float* tmp, float* d_out, float* acc,
                        const feat_reduce_ws_t* ws);
+/* The producers of a smoother's first iterate in FP32 (as feat_defect_first_f64 and the
+ * others there); feat_convert_first_f64_f32: feat_convert_f64_f32 + x1 of the smoother on
+ * the converted vector, filtered through `mask` (x1 may not be o). */
+int feat_convert_first_f64_f32(feat_handle_t h, float* o, const double* in, uint64_t n,
+                               const float* inv_diag, const uint32_t* mask, float omega, float* x1);
+int feat_apply_masked_first_f32(feat_handle_t h, const feat_matrix_f32_t* A, float* r, const float* x,
+                                const uint32_t* mask, double* nrm2, const float* inv_diag,
+                                float omega, float* x1, const feat_reduce_ws_t* ws);
+int feat_defect_first_f32(feat_handle_t h, const feat_matrix_f32_t* A, float* d, const float* rhs,
+                          const float* x, const uint32_t* mask, double* nrm2, const float* inv_diag,
+                          float omega, float* x1, const feat_reduce_ws_t* ws);
+int feat_rj_smooth_from1_f32(feat_handle_t h, const feat_matrix_f32_t* A, const float* inv_diag,
+                             const uint32_t* mask, int steps, float omega, const float* rhs,
+                             const double* rhs_nrm2, float* x, float* tmp, float* d_out, float* acc,
+                             const feat_reduce_ws_t* ws);
 int feat_dense_gemv_f32(feat_handle_t h, int n, const float* ainv, const float* b, float* x,
                         const uint32_t* mask);
 /* ConvertPrecond's way back: z = double(z32) and *dot = z . w in FP64. */

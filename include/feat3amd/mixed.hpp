@@ -319,20 +319,39 @@ namespace feat3amd
         auto nrm_of = [&](Index i) -> const double* { return i == 0 ? def_nrm2 : _fw.scalar(2 + i); };
         if(!_tail_built) _build_tail();
         const Index t = _tail_t ? _tail_t : c;   // levels from t down run in the fused tail (when _tail_t)
-        check(feat_convert_f64_f32(hd, _l[0].rhs.elements(), (const double*)def.elements(), def.size()), "to FP32");
+        // every smoother above the fused levels (of two or more steps) starts from the iterate
+        // formed by the kernel that produced its right-hand side: the conversion, the restriction
+        // or the defect after the prolongation
+        auto x1_at = [&](Index i, int steps, float* x) -> float* {
+          return steps < 2 ? nullptr : (steps & 1) ? x : _l[i].tmp.elements();
+        };
+        auto pre_x1 = [&](Index i) { return i < t ? x1_at(i, _l[i].pre_steps, _l[i].sol.elements()) : nullptr; };
+        if(float* x1 = pre_x1(0))
+          check(feat_convert_first_f64_f32(hd, _l[0].rhs.elements(), (const double*)def.elements(), def.size(),
+                                           _l[0].inv_pre.elements(), _h->levels[0].filter->mask(), _l[0].omega_pre, x1),
+                "to FP32");
+        else
+          check(feat_convert_f64_f32(hd, _l[0].rhs.elements(), (const double*)def.elements(), def.size()), "to FP32");
         for(Index i = 0; i < t; ++i)
         {
           auto& lv = _h->levels[i];
           Level32& l = _l[i];
           const feat_matrix_f32_t& A = plan(*lv.matrix);
-          check(feat_rj_smooth_f32(hd, &A, l.inv_pre.elements(), lv.filter->mask(), l.pre_steps, l.omega_pre,
-                                   l.rhs.elements(), nrm_of(i), l.sol.elements(), l.tmp.elements(), l.def.elements(),
-                                   nullptr, ws),
+          auto smooth = pre_x1(i) ? feat_rj_smooth_from1_f32 : feat_rj_smooth_f32;
+          check(smooth(hd, &A, l.inv_pre.elements(), lv.filter->mask(), l.pre_steps, l.omega_pre,
+                       l.rhs.elements(), nrm_of(i), l.sol.elements(), l.tmp.elements(), l.def.elements(),
+                       nullptr, ws),
                 "FP32 pre-smoothing");
           const feat_matrix_f32_t& R = _rest(i);
-          check(feat_apply_masked_f32(hd, &R, _l[i + 1].rhs.elements(), l.def.elements(), _h->levels[i + 1].filter->mask(),
-                                      _tail_t && i + 1 == t ? nullptr : _fw.scalar(2 + i + 1), ws),
-                "FP32 restriction");
+          Level32& lc = _l[i + 1];
+          if(float* x1 = pre_x1(i + 1))
+            check(feat_apply_masked_first_f32(hd, &R, lc.rhs.elements(), l.def.elements(), _h->levels[i + 1].filter->mask(),
+                                              _fw.scalar(2 + i + 1), lc.inv_pre.elements(), lc.omega_pre, x1, ws),
+                  "FP32 restriction");
+          else
+            check(feat_apply_masked_f32(hd, &R, lc.rhs.elements(), l.def.elements(), _h->levels[i + 1].filter->mask(),
+                                        _tail_t && i + 1 == t ? nullptr : _fw.scalar(2 + i + 1), ws),
+                  "FP32 restriction");
         }
         if(_tail_t)
           check(feat_mg_tail_f32(hd, &_tail, _l[t].rhs.elements(), nullptr, _l[t].sol.elements()),
@@ -377,10 +396,17 @@ namespace feat3amd
           check(feat_prol_add_f32(hd, &P, l.sol.elements(), _l[k + 1].sol.elements(), lv.filter->mask()), "FP32 prolongation");
           const feat_matrix_f32_t& A = plan(*lv.matrix);
           double* dn = _fw.scalar(2 + L + k);
-          check(feat_defect_f32(hd, &A, l.def.elements(), l.rhs.elements(), l.sol.elements(), lv.filter->mask(), dn, ws),
-                "FP32 defect");
-          check(feat_rj_smooth_f32(hd, &A, l.inv_post.elements(), lv.filter->mask(), l.post_steps, l.omega_post,
-                                   l.def.elements(), dn, l.cor.elements(), l.tmp.elements(), nullptr, l.sol.elements(), ws),
+          float* x1 = x1_at(k, l.post_steps, l.cor.elements());
+          if(x1)
+            check(feat_defect_first_f32(hd, &A, l.def.elements(), l.rhs.elements(), l.sol.elements(), lv.filter->mask(), dn,
+                                        l.inv_post.elements(), l.omega_post, x1, ws),
+                  "FP32 defect");
+          else
+            check(feat_defect_f32(hd, &A, l.def.elements(), l.rhs.elements(), l.sol.elements(), lv.filter->mask(), dn, ws),
+                  "FP32 defect");
+          auto smooth = x1 ? feat_rj_smooth_from1_f32 : feat_rj_smooth_f32;
+          check(smooth(hd, &A, l.inv_post.elements(), lv.filter->mask(), l.post_steps, l.omega_post,
+                       l.def.elements(), dn, l.cor.elements(), l.tmp.elements(), nullptr, l.sol.elements(), ws),
                 "FP32 post-smoothing");
         }
         check(feat_convert_dot_f32_f64(hd, (double*)cor.elements(), _l[0].sol.elements(), (const double*)def.elements(),
