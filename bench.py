@@ -536,6 +536,16 @@ def read_ceilings(feat, torch, dev, stream, h, nbytes, reps):
     return out
 
 
+def diag_plan_bytes(m):
+    """Bytes a launch needs of a diagonal plan: where its interior rows are one stencil
+    (grid_n1), the stencil and the code words of the boundary rows; else one byte per offset
+    slot; and the pair table."""
+    if m.grid_n1:
+        m1 = int(m.grid_n1)
+        return (m1 ** DIM - (m1 - 2) ** DIM) * 4 * int(m.slice_words) + 27 * 8 + 256 * 12
+    return int(m.nnz) + 256 * 12
+
+
 def spmv_only(feat, torch, dev, stream, args):
     """SpMV r = A*x on the level-7 matrix in each format, args.spmv_reps launches each,
     then args.spmv_reps device-to-device copies of 1 GiB (the counter calibration)."""
@@ -578,7 +588,7 @@ def spmv_only(feat, torch, dev, stream, args):
     e1.synchronize()
     out["jacobi_step_us"] = e0.elapsed_time(e1) * 1e3 / args.spmv_reps
     log(f"jacobi step: {out['jacobi_step_us']:.1f} us per launch")
-    out["read_ceiling"] = read_ceilings(feat, torch, dev, stream, h, int(dm.nnz) + 256 * 12 + 4 * n * 8, args.spmv_reps)
+    out["read_ceiling"] = read_ceilings(feat, torch, dev, stream, h, diag_plan_bytes(dm) + 4 * n * 8, args.spmv_reps)
     src = torch.empty(1 << 27, dtype=torch.float64, device=dev)
     dst = torch.empty_like(src)
     src.fill_(1.0)
@@ -870,23 +880,24 @@ def main():
     # measured read ceilings (feat_stream_read_f64): a buffer of the Jacobi step's bytes read
     # again and again (held in the last-level cache like the step's own arrays), and the same
     # bytes from HBM (eight such windows of a larger buffer in turn)
-    ceil = read_ceilings(feat, torch, dev, stream, h, int(dplan.nnz) + 256 * 12 + 4 * n * 8, args.spmv_reps)
+    plan_bytes = diag_plan_bytes(dplan)
+    ceil = read_ceilings(feat, torch, dev, stream, h, plan_bytes + 4 * n * 8, args.spmv_reps)
     idx_bytes = {feat.IDX_D16: 2, feat.IDX_U32: 4}[plan.index]
     nslices = (n + 63) // 64
     # bytes each kernel must move: its own arrays once, x once, r once
     csr_bytes = spmv_bytes(n, nnz)
     sell_bytes = int(plan.nnz) * (8 + idx_bytes) + n * 2 + (nslices + 1) * 8 + 2 * n * 8
     # pair dictionary in entry order: one byte per stored entry, row lengths, slice offsets,
-    # the 3 KB pair table, x, r; by diagonal: one byte per slot (27 per row), the table, x, r
+    # the 3 KB pair table, x, r; by diagonal: the plan's bytes, x, r
     edict_bytes = int(eplan.nnz) + n * 2 + (nslices + 1) * 8 + 256 * 12 + 2 * n * 8
-    dict_bytes = int(dplan.nnz) + 256 * 12 + 2 * n * 8
+    dict_bytes = plan_bytes + 2 * n * 8
     edict_gbs = edict_bytes / (edict_ms * 1e-3) / 1e9
     csr_gbs = csr_bytes / (csr_ms * 1e-3) / 1e9
     sell_gbs = sell_bytes / (sell_ms * 1e-3) / 1e9
     dict_gbs = dict_bytes / (dict_ms * 1e-3) / 1e9
     # Jacobi step: the plan's bytes, x_k (gathered and read by the epilogue: once), rhs,
     # inverse diagonal, x_{k+1}
-    step_bytes = int(dplan.nnz) + 256 * 12 + 4 * n * 8
+    step_bytes = plan_bytes + 4 * n * 8
     step_gbs = step_bytes / (step_ms * 1e-3) / 1e9
     log(f"jacobi step on the diagonal plan: {step_ms * 1e3:.1f} us, {step_gbs:.0f} GB/s")
     ref_model = nnz * 16 + n * 8             # product_matvec-bench.cpp:41-44 model (GiB = 1024^3)
@@ -927,7 +938,7 @@ def main():
             "other_plans_rel_diff_x": plan_rel_diff,
             "default_launch_shapes_s_per_solve": t_untuned,
             "matrix_plan": "SELL-64 pair dictionary by diagonal (1 byte per offset slot, 9 triples of offsets, "
-                           "42 distinct (col-row, value) pairs)",
+                           "42 distinct (col-row, value) pairs), interior rows from one stencil",
             "parallelism": "single GPU",
         },
         "mixed_precision": {"form": "FP32 V-cycle on FP32 / FP16-valued SELL-64 plans (FP64 coarse solve) "
@@ -939,10 +950,10 @@ def main():
                                     "the transfer operators in FP16 and uses the FP32 dictionary elsewhere",
                             "variable_coefficient_level7": mixed_vc},
         "spmv": {
-            "sell64_diag": {"kernel": "k_sell_diag_rows<double,EpiApply<double>>", "us_per_launch": dict_ms * 1e3,
+            "sell64_diag": {"kernel": "k_sten_rows<double,EpiApply<double>,3,3>", "us_per_launch": dict_ms * 1e3,
                             "bytes_per_launch": dict_bytes, "gbps": dict_gbs,
                             "csr_equivalent_gbps": csr_bytes / (dict_ms * 1e-3) / 1e9,
-                     "jacobi_step": {"kernel": "k_sell_diag_rows<double,EpiSmooth<double>> (one fused "
+                     "jacobi_step": {"kernel": "k_sten_rows<double,EpiSmooth<double>,3,3> (one fused "
                                                "Richardson(Jacobi) step, the solve's most frequent launch)",
                                      "us_per_launch": step_ms * 1e3, "achieved": step_gbs,
                                      "frac": step_gbs / PEAK_HBM_GBS, "algorithmic_bytes": step_bytes}, "stored_slots": dict_padded},
@@ -965,10 +976,10 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS, "traffic": SPMV_TRAFFIC_BYTES["jacobi_step"],
                      "algorithmic_bytes": step_bytes, "us_per_launch": step_ms * 1e3,
-                     "kernel": "k_sell_diag_rows<double,EpiSmooth<double>,9,7>: one fused Richardson(Jacobi) "
+                     "kernel": "k_sten_rows<double,EpiSmooth<double>,3,3>: one fused Richardson(Jacobi) "
                                "step x_{k+1} = x_k + 0.5 filter(inv_diag (rhs - A x_k)) on the level-7 diagonal "
-                               "pair-dictionary plan (the solve's dominant kernel: 35 of its launches per solve), "
-                               "bytes = codes (1 B per offset slot, 27 slots in 7 words per row) + pair table + "
+                               "pair-dictionary plan with uniform interior rows (the solve's dominant kernel: 35 "
+                               "of its launches per solve), bytes = stencil + code words of the boundary rows + "
                                "x_k + rhs + inv_diag + x_{k+1}",
                      "measured_read_ceiling": ceil,
                      "frac_of_read_ceiling_same_bytes": achieved / ceil["same_bytes_repeated_gbps"],

@@ -3615,8 +3615,8 @@ constexpr int kTailSmoothed = FEAT_MG_TAIL_MAX_LEVELS - 1;
 //    row's 3^dim values stay in registers for the 4 or 5 sweeps of a leg, so a leg reads them
 //    once from the caches, and only for free rows; a kernel per dimension keeps them out of
 //    scratch (with the dimension at run time a third of them went there: 63 us instead of 37).
-//    729 + 125 rows over a direct 27, V(4,4): 37 us in FP64, 32 us in FP32 with FP16 values,
-//    against about 110 us of 25 launches.
+//    729 + 125 rows over a direct 27, V(4,4): 37 us in FP64, 30 us in FP32 with FP16 values,
+//    against about 100 us of 25 launches.
 enum TailMode { kTailPlan, kTailGrid, kTailBand2, kTailBand3 };
 template<typename DT, int MODE>
 struct TailRow
