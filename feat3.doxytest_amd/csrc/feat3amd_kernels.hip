@@ -1567,6 +1567,18 @@ __global__ void k_sten_check(const uint32_t* codes, uint32_t nw, uint32_t nslot,
   }
 }
 
+// The stencil of the interior rows, from row ref's codes (at most 27 slots, one lane each).  Formed
+// on the device: read back with a strided copy into pageable memory, the code words were still
+// zero after the stream's synchronisation in the first plan of a process run under a kernel
+// trace, and the stencil with them.
+template<typename DT>
+__global__ void k_sten_values(const uint32_t* codes, uint32_t nw, uint32_t nslot, uint64_t ref, const DT* tab, DT* sten)
+{
+  const uint32_t* rw = codes + (ref >> 6) * 64 * nw + (ref & 63);
+  const uint32_t t = threadIdx.x;
+  if(t < nslot) sten[t] = tab[(rw[(t >> 2) * 64] >> (8 * (t & 3))) & 255u];
+}
+
 // Pair-dictionary construction.  Distinct value bit patterns and distinct
 // column - row offsets are collected in two open-addressing tables of
 // kDictSlots keys (relaxed reads first, compare-and-swap only to insert); the
@@ -2775,19 +2787,16 @@ int dict_create(feat_handle_t h, const feat_csr_f64_t* A, const std::vector<uint
       if(rc) break;
       hipLaunchKernelGGL(k_sten_check, dim3(grid_for(n)), dim3(kThreads), 0, h->stream, codes, dw, uint32_t(nslot),
                          int(d), uint32_t(q), n, ref, (int*)state);
-      std::vector<uint32_t> words_of(dw);
       rc = check_launch(name);
       if(!rc) rc = check_hip(hipMemcpyAsync(&bad, state, sizeof(uint32_t), hipMemcpyDeviceToHost, h->stream), "copy");
-      if(!rc)
-        rc = check_hip(hipMemcpy2DAsync(words_of.data(), sizeof(uint32_t), codes + (ref >> 6) * 64 * dw + (ref & 63),
-                                        64 * sizeof(uint32_t), sizeof(uint32_t), dw, hipMemcpyDeviceToHost, h->stream), "copy");
       if(!rc) rc = check_hip(hipStreamSynchronize(h->stream), "sync");
       if(rc || bad) break;
-      std::vector<DT> sv(nslot);
-      for(uint64_t t = 0; t < nslot; ++t) sv[t] = tv[(words_of[t >> 2] >> (8 * (t & 3))) & 255u];
-      rc = check_hip(hipMemcpyAsync(reinterpret_cast<char*>(table) + sten_offset<DT>(), sv.data(), sizeof(DT) * nslot,
-                                    hipMemcpyHostToDevice, h->stream), "copy");
+      hipLaunchKernelGGL((k_sten_values<DT>), dim3(1), dim3(64), 0, h->stream, codes, dw, uint32_t(nslot), ref,
+                         reinterpret_cast<const DT*>(table),
+                         reinterpret_cast<DT*>(reinterpret_cast<char*>(table) + sten_offset<DT>()));
+      rc = check_launch(name);
       if(!rc) rc = check_hip(hipStreamSynchronize(h->stream), "sync");
+      if(rc) break;
       grid_n1 = uint32_t(q);
       grid_dim = d;
     }
