@@ -33,11 +33,11 @@ PEAK_HBM_GBS = 8000.0
 # `bench.py --spmv-only` (FETCH_SIZE, then WRITE_SIZE, KiB per dispatch); FETCH_SIZE is scaled
 # by 2.0 and WRITE_SIZE by 1.0, the factors that make the same counters read 1 GiB for a
 # 1 GiB device-to-device copy (profiles/spmv_traffic_3d_q1_l7.md)
-SPMV_TRAFFIC_BYTES = {"jacobi_step": 55483.9 * 2048 + 16771.0 * 1024,
-                      "sell64_diag": 38712.2 * 2048 + 16771.0 * 1024,
-                      "sell64_dict": 40575.7 * 2048 + 16771.0 * 1024,
-                      "sell64": 295808.9 * 2048 + 16771.0 * 1024,
-                      "csr_u64": 474623.3 * 2048 + 16771.0 * 1024}
+SPMV_TRAFFIC_BYTES = {"jacobi_step": 43510.0 * 2048 + 17442.0 * 1024,
+                      "sell64_diag": 22458.0 * 2048 + 17457.0 * 1024,
+                      "sell64_dict": 40574.2 * 2048 + 16771.0 * 1024,
+                      "sell64": 295825.0 * 2048 + 16771.0 * 1024,
+                      "csr_u64": 475394.0 * 2048 + 16771.0 * 1024}
 
 
 def load_feat():
