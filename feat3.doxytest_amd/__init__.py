@@ -51,7 +51,7 @@ class Matrix(C.Structure):
     _fields_ = [("format", _i), ("index", _i), ("rows", _u64), ("cols", _u64), ("nnz", _u64),
                 ("val", _vp), ("col", _vp), ("ptr", _vp), ("rowlen", _vp), ("value_kind", _i),
                 ("scale", _f), ("tune", _i), ("slice_words", C.c_uint32), ("grid_n1", C.c_uint32),
-                ("grid_dim", C.c_uint32)]
+                ("grid_dim", C.c_uint32), ("grid_closed", C.c_uint32)]
 
 
 FMT_CSR, FMT_SELL, FMT_DLINEAR, FMT_BANDED = 0, 1, 2, 3

@@ -785,7 +785,10 @@ __global__ __launch_bounds__(kThreads) void k_sell_diag_rows(const DT* __restric
 // Positions are flat in the plane, so the values at a plane's edges are of the wrong row; the
 // rows they belong to are boundary rows.  A boundary row that the epilogue filters does not
 // use its sum and is finished in place; the others are summed from their codes at the end, one
-// lane per boundary row.
+// lane per boundary row.  Those rows come after the march, with scattered loads of their own, and
+// cost a small 3D grid more than the march gains: sten_marches.  Nine loads at a time (one at a
+// time, each behind its code's branch, a smoother call of 4 steps with no filter took 67 us instead of
+// 51 on 97^3 nodes in FP64, 28 instead of 25 on 513^2; 91 instead of 97 on 129^3).
 __host__ __device__ inline uint32_t grid_boundary_rows(int dim, uint32_t n1)
 {
   return dim == 3 ? 2 * n1 * n1 + (n1 - 2) * (4 * n1 - 4) : 4 * n1 - 4;
@@ -897,17 +900,56 @@ __global__ __launch_bounds__(kThreads) void k_sten_rows(const DT* __restrict__ t
     const typename Epi::Pre pf = epi.pre(row);
     if(epi.filtered(pf)) continue;   // finished in place
     const uint32_t* cw = codes + uint64_t(row >> 6) * 64 * NW + (row & 63);
-    DT sum = DT(0);
+    uint32_t w[NW];
 #pragma unroll
-    for(int t = 0; t < 3 * NT; ++t)
+    for(int k = 0; k < NW; ++k) w[k] = cw[64 * k];
+    DT sum = DT(0);
+    auto code = [&](int t) { return (w[t >> 2] >> (8 * (t & 3))) & 255u; };
+    auto place = [&](int t) { return t % 3 - 1 + (DIM == 3 ? (t / 3) % 3 - 1 : t / 3 - 1) * m + (DIM == 3 ? t / 9 - 1 : 0) * P; };
+#pragma unroll
+    for(int t0 = 0; t0 < 3 * NT; t0 += 9)
     {
-      const uint32_t c = (cw[(t >> 2) * 64] >> (8 * (t & 3))) & 255u;
-      const int dx = t % 3 - 1, dy = DIM == 3 ? (t / 3) % 3 - 1 : t / 3 - 1, dz = DIM == 3 ? t / 9 - 1 : 0;
-      if(c != kDiagNone) sum = dfma(tab[c], x[int32_t(row) + dx + dy * m + dz * P], sum);
+      // nine taps' loads together, unconditional (an empty slot reads the row's own place)
+      // unless all nine are outside the grid; the barriers keep the compiler from holding more
+      // of them, whose registers would cost the march a wave
+      bool any = false;
+#pragma unroll
+      for(int t = t0; t < t0 + 9; ++t) any = any || code(t) != kDiagNone;
+      if(!any) continue;
+      DT av[9], xv[9];
+#pragma unroll
+      for(int k = 0; k < 9; ++k)
+      {
+        av[k] = tab[code(t0 + k)];
+        xv[k] = x[int32_t(row) + (code(t0 + k) != kDiagNone ? place(t0 + k) : 0)];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for(int k = 0; k < 9; ++k)
+      {
+        const DT s = dfma(av[k], xv[k], sum);
+        sum = code(t0 + k) != kDiagNone ? s : sum;
+      }
+      __builtin_amdgcn_sched_barrier(0);
     }
     epi.row(row, sum, pf, acc0, acc1);
   }
   grid_reduce_finish(gr, acc0, acc1);
+}
+
+// Whether a uniform-stencil plan marches.  In 2D always.  In 3D where the caller has said that every
+// boundary row is filtered (grid_closed), or from kStenOpen one-plane workgroups on (97^3 nodes);
+// smaller grids keep the code words otherwise, as the mask may leave boundary rows to sum.  A
+// smoother call of 4 steps in FP64, code words / march: 33^3 nodes filtered 18 / 18 us, open
+// 17 / 28; 65^3 filtered 28 / 27, open 26 / 37; 97^3 filtered 64 / 51, open 58 / 51; 129^3
+// filtered 121 / 83, open 109 / 97.  2D, 513^2 filtered 26 / 22, open 26 / 25.
+constexpr uint64_t kStenOpen = 3584;
+template<class M>
+bool sten_marches(const M* A)
+{
+  if(A->grid_dim != 3 || A->grid_closed) return true;
+  const uint64_t n1 = A->grid_n1;
+  return (n1 * n1 + kHaloChunk - 1) / kHaloChunk * n1 >= kStenOpen;
 }
 
 // the march of a uniform-stencil plan
@@ -1239,7 +1281,7 @@ int launch_mat(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gri
       finish_reduce(s, gd, uint64_t(grid));
       return check_launch(name);
     }
-    if(A->index == FEAT_IDX_DIAG && A->grid_n1) return launch_sten<DT>(s, A, x, epi, gr, name);
+    if(A->index == FEAT_IDX_DIAG && A->grid_n1 && sten_marches(A)) return launch_sten<DT>(s, A, x, epi, gr, name);
     if(A->index == FEAT_IDX_DIAG)
     {
       // chunks of kHaloChunk rows (62 per wave); a dot or norm is summed per chunk, so it

@@ -286,6 +286,10 @@ typedef struct {
                                 every interior row.  FEAT_FMT_BANDED: the values are
                                 symmetric bit for bit                         */
   uint32_t grid_dim;
+  uint32_t grid_closed;      /* FEAT_IDX_DIAG with grid_n1: 1 where every boundary node
+                                of the grid is filtered in the calls with this
+                                descriptor (the caller's hint for the launch shape;
+                                the results do not depend on it)              */
 } feat_matrix_f64_t;
 
 typedef struct {             /* FP32 arithmetic (mixed-precision inner solver) */
@@ -299,7 +303,7 @@ typedef struct {             /* FP32 arithmetic (mixed-precision inner solver) *
   float scale;               /* row sums are multiplied by this power of two  */
   int tune;                  /* SELL launch shape, 0 = default                */
   uint32_t slice_words;      /* as feat_matrix_f64_t::slice_words             */
-  uint32_t grid_n1, grid_dim;   /* as feat_matrix_f64_t                       */
+  uint32_t grid_n1, grid_dim, grid_closed;   /* as feat_matrix_f64_t          */
 } feat_matrix_f32_t;
 
 /* A CSR descriptor (no copy) of the caller's arrays. */

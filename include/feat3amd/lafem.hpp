@@ -354,6 +354,15 @@ namespace feat3amd
 
       bool has_plan() const { return bool(_plan); }
 
+      /// Tells the plans made so far whether the filter they are used with holds every boundary
+      /// node of the grid (grid_closed: a hint for the launch shape of uniform stencils).
+      void set_boundary_filtered(bool on) const
+      {
+        if(_plan) _plan->grid_closed = on ? 1u : 0u;
+        if(_plan32) _plan32->grid_closed = on ? 1u : 0u;
+        if(_plan16) _plan16->grid_closed = on ? 1u : 0u;
+      }
+
       /// Picks the fastest launch shape of the execution plan's row kernels
       /// (feat_autotune_matrix_f64; bit-identical results for every shape).
       /// Returns the time per SpMV of the chosen shape in microseconds (-1: nothing to tune).

@@ -284,6 +284,7 @@ namespace feat3amd
           L->cor.component_invert(L->inv, 1.0);             // coarsest level: 1 / a_ii
           L->inv.component_invert(L->inv, _cfg.omega_jac);  // omega / a_ii
           (void)L->A.exec();
+          L->A.set_boundary_filtered(true);   // unit_mask(q1_boundary) above
           if(k > Lc)
           {
             (void)L->P.exec();

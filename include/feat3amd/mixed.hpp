@@ -65,6 +65,7 @@ namespace feat3amd
           const bool cand = s >= 1 && lv.matrix->rows() <= FEAT_MG_TAIL_MAX_ROWS;
           _grid[s] = tail_grid_form(*lv.matrix, lv.filter->mask(), lv.transfer->get_mat_prol(),
                                     lv.transfer->get_mat_rest(), _h->levels[s + 1].matrix->rows(), cand);
+          lv.matrix->set_boundary_filtered(_grid[s].closed);
           if(!_grid[s].sten.empty())
           {
             std::vector<float> s32(_grid[s].sten.begin(), _grid[s].sten.end());

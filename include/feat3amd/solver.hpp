@@ -413,13 +413,14 @@ namespace feat3amd
     ///    descriptors, and in the fused coarse levels as feat_mg_tail_level_t dlinear.
     ///  * sten (fused coarse levels only): every free row (not in the mask) holds the same
     ///    3^dim values at the neighbour offsets in CSR order (feat_mg_tail_level_t sten).
-    /// Both are checked entry by entry on host copies of the matrices.
+    ///  * closed: the filter holds every boundary node of the grid.
+    /// All are checked entry by entry on host copies of the matrices and the filter's mask.
     struct TailGridForm
     {
       int dim = 0;
       std::uint32_t n1 = 0;
       std::vector<double> sten;   // empty: the rows come from the plan
-      bool dlinear = false;
+      bool dlinear = false, closed = false;
     };
 
     template<typename Matrix_>
@@ -445,7 +446,7 @@ namespace feat3amd
           }
         }
       }
-      if(!dim || !Runtime::grid_forms()) return f;
+      if(!dim) return f;
       f.dim = dim;
       f.n1 = std::uint32_t(n1);
       auto down = [](auto* dst, const auto* src, std::size_t count) {
@@ -462,10 +463,13 @@ namespace feat3amd
       };
       std::vector<double> av, pv, rv;
       std::vector<std::uint64_t> ac, ap, pc, pp, rc, rp;
-      if(want_stencil) fetch(A, av, ac, ap);
-      fetch(P, pv, pc, pp);
-      fetch(R, rv, rc, rp);
-      std::vector<std::uint32_t> mask(want_stencil && mask_dev ? (n + 31) / 32 : 0, 0u);
+      if(Runtime::grid_forms())
+      {
+        if(want_stencil) fetch(A, av, ac, ap);
+        fetch(P, pv, pc, pp);
+        fetch(R, rv, rc, rp);
+      }
+      std::vector<std::uint32_t> mask(mask_dev ? (n + 31) / 32 : 0, 0u);
       down(mask.data(), mask_dev, mask.size());
       Runtime::synchronize();
       const std::int64_t nn = n1 * n1, nc = (n1 + 1) / 2;
@@ -475,6 +479,16 @@ namespace feat3amd
         y = (i / side) % side;
         z = dim == 3 ? i / (side * side) : 0;
       };
+      f.closed = !mask.empty();
+      for(std::int64_t i = 0; i < std::int64_t(n) && f.closed; ++i)
+      {
+        std::int64_t x, y, z;
+        coord(i, n1, x, y, z);
+        if((x == 0 || x == n1 - 1 || y == 0 || y == n1 - 1 || (dim == 3 && (z == 0 || z == n1 - 1))) &&
+           !((mask[i >> 5] >> (i & 31)) & 1u))
+          f.closed = false;
+      }
+      if(!Runtime::grid_forms()) return f;   // closed whatever the forms: the rows' kernels depend on it
       // the stencil of the free rows
       bool sten_ok = want_stencil;
       for(std::int64_t i = 0; i < std::int64_t(n) && sten_ok; ++i)
@@ -687,6 +701,7 @@ namespace feat3amd
           const bool cand = s >= 1 && l.matrix->rows() <= FEAT_MG_TAIL_MAX_ROWS;
           _grid[s] = tail_grid_form(*l.matrix, l.filter->mask(), l.transfer->get_mat_prol(), l.transfer->get_mat_rest(),
                                     _h->levels[s + 1].matrix->rows(), cand);
+          l.matrix->set_boundary_filtered(_grid[s].closed);
           if(!_grid[s].sten.empty())
             _grid_sten[s] = DeviceArray<double>::from_host(_grid[s].sten.data(), _grid[s].sten.size());
           if(_grid[s].dlinear)

@@ -1,7 +1,9 @@
 """Diagonal plans of structured grids whose interior rows are all the same (the march over planes):
 the rows equal the entry-order dictionary plan's bit for bit at grid sizes around the 62 positions
 a wave covers and the planes a lane takes, with no filter, with the boundary filtered, and with
-some boundary and interior rows filtered; a grid with one odd interior row keeps the code words."""
+some boundary and interior rows filtered; a grid with one odd interior row keeps the code words.
+3D grids below 97 nodes a side march with the descriptor's grid_closed only (a hint: the results are
+those of the code words whether the boundary is filtered or not)."""
 import itertools
 
 import numpy as np
@@ -32,7 +34,7 @@ def grid_csr(dim, n1, odd_row=False):
 
 
 @pytest.mark.parametrize("dim,n1", [(2, 3), (2, 9), (2, 61), (2, 62), (2, 63), (2, 64), (2, 249), (2, 1100), (3, 3), (3, 4),
-                                    (3, 7), (3, 8), (3, 16), (3, 33), (3, 64), (3, 65)])
+                                    (3, 7), (3, 8), (3, 16), (3, 33), (3, 64), (3, 65), (3, 96), (3, 97)])
 def test_march_bitwise(feat, handle, torch_gpu, dim, n1):
     print(f"stencil march dim={dim} n1={n1}", flush=True)
     torch = torch_gpu
@@ -47,7 +49,9 @@ def test_march_bitwise(feat, handle, torch_gpu, dim, n1):
     for fp in ("f64", "f32"):
         dt = torch.float64 if fp == "f64" else torch.float32
         x, rhs, inv = (torch.from_numpy(rng.standard_normal(n)).cuda().to(dt) for _ in range(3))
-        plans = [feat.SellPlan(handle, *dev, n, n, fp=fp), feat.SellPlan(handle, *dev, n, n, fp=fp, diag=False)]
+        plans = [feat.SellPlan(handle, *dev, n, n, fp=fp), feat.SellPlan(handle, *dev, n, n, fp=fp, diag=False),
+                 feat.SellPlan(handle, *dev, n, n, fp=fp)]
+        plans[0].m.grid_closed = 1
         # plans whose empty slots exceed a quarter of the entries keep the entry-order dictionary
         diag = -(-n // 64) * 64 * 3 ** dim <= val.size + val.size // 4 + 64 * 3 ** dim
         assert plans[0].m.index == (feat.IDX_DIAG if diag else feat.IDX_DICT)
@@ -75,10 +79,11 @@ def test_march_bitwise(feat, handle, torch_gpu, dim, n1):
                     feat.check(k.feat_apply_masked_f32(handle.h, pl.m, P(o[2]), P(x), P(mask), None, ws), "apply")
                 handle.sync()
                 out.append((o, float(s[0])))
-            for a, b in zip(out[0][0], out[1][0]):
-                assert torch.equal(a, b), (fp, filt is None)
+            for a, b, c in zip(out[0][0], out[1][0], out[2][0]):
+                assert torch.equal(a, b) and torch.equal(c, b), (fp, filt is None)
             # the norm is the same sum in another order
             assert abs(out[0][1] - out[1][1]) <= 1e-13 * out[1][1]
+            assert abs(out[2][1] - out[1][1]) <= 1e-13 * out[1][1]
         for pl in plans:
             pl.close()
 
