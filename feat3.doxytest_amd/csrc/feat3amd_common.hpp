@@ -41,7 +41,6 @@ constexpr int kThreads = 256;
 constexpr int kXcd = 8;
 constexpr int kMaxGrid = FEAT_REDUCE_MAX_BLOCKS;
 constexpr int kRowsPerBlock = 256;  // rows per CSR row-block (one lane per row)
-constexpr uint64_t kCsrStream = 6144;   // CSR row-blocks from which a matrix streams from HBM
 constexpr int kSellUnroll = 8;      // SELL entries per row in flight
 
 

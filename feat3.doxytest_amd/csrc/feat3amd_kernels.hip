@@ -98,10 +98,13 @@ struct EpiCentre<E, DT, std::void_t<decltype(std::declval<const E&>().pre(uint64
 // in flight.  One pass after the other (load, gather, store, barrier, add, barrier) a block of
 // ragged rows was one long chain of round trips: 300 k rows of 0 to 40 entries, FP32, 31 us;
 // now 26 us, bound by the 64 cache lines of each scattered gather.  50 k such rows 22.7 -> 9 us
-// (FP64, 64-bit columns 19.5 -> 12), 3D Q1 level 5 18.6 -> 11.4 us; level 7, which streams 982 MB
-// at the rate of a copy, does without (PIPE false; launch_rows).
+// (FP64, 64-bit columns 19.5 -> 12), 3D Q1 level 5 18.6 -> 11.4 us.  Matrices of short rows, and
+// 3D Q1 level 7, which streams 982 MB at the rate of a copy (188 us plain, 200 pipelined), do
+// without (PIPE false): csr_pipelined.
 // ---------------------------------------------------------------------------
-template<typename DT, typename IT, class Epi, int U, bool PIPE>
+// UNR: the sums of the plain passes unrolled by four (27 entries a row: 2 % faster; 2 entries a
+// row: 5 to 10 % slower).
+template<typename DT, typename IT, class Epi, int U, bool PIPE, bool UNR>
 __global__ __launch_bounds__(kThreads) void k_csr_rows(const DT* __restrict__ val,
                                                        const IT* __restrict__ col,
                                                        const IT* __restrict__ rowptr,
@@ -171,7 +174,14 @@ __global__ __launch_bounds__(kThreads) void k_csr_rows(const DT* __restrict__ va
           s_x[0][t + u * kThreads] = xv[u];
         }
         __syncthreads();
-        add(c0, 0);
+        if constexpr(UNR)
+          add(c0, 0);
+        else if(mine)
+        {
+          const uint64_t kb = rs > c0 ? rs : c0;
+          const uint64_t ke = re < c0 + cn ? re : c0 + cn;
+          for(uint64_t k = kb; k < ke; ++k) sum = dfma(s_val[0][k - c0], s_x[0][k - c0], sum);
+        }
         __syncthreads();
       }
     }
@@ -442,23 +452,44 @@ struct EpiSmooth
   __device__ __forceinline__ void row(uint64_t i, DT sum, double& a0, double& a1) const { row(i, sum, pre(i), a0, a1); }
 };
 
+// Whether the rows of a CSR matrix take the pipelined passes, from its mean row length (10, 16, ..
+// entries): the pipeline pays where a block has several passes to hide, and costs its unneeded
+// loads past a block's end where it has one or two.  Plain / pipelined time of one apply, rows of
+// 0 to twice the mean with columns near the diagonal to spread over a hundredth of the width:
+//                      8 entries a row  10          16          20          27          40
+//   70 k rows,  16 B   0.97 .. 1.01     1.02-1.07   1.28-1.32   1.38-1.47   1.62-1.70   1.81-1.86
+//   300 k,      16 B   0.77 .. 0.94     0.80-1.00   0.93-1.09   0.99-1.13   1.10-1.16   1.13-1.18
+//   1 M,        16 B   0.81 .. 1.01     0.84-1.03   0.95-1.09   0.96-1.12   0.99-1.15   1.06-1.18
+//   1 M,   f64+u32     0.89 .. 1.02     0.92-1.06   1.05-1.15   1.10-1.17   1.17-1.20   1.20
+//   1 M,   f32+u32     0.84 .. 1.08     0.84-1.09   1.06-1.21   1.15-1.25   1.28-1.30   1.38-1.54
+//   1 M,   f32+u64     0.76 .. 1.04     0.76-1.04   0.94-1.20   1.02-1.21   1.12-1.28   1.34-1.38
+// and 0.5 to 0.9 with 2 to 5 entries a row.  The lines lie where no kind of columns loses: 10
+// entries while the blocks leave the chip room (512), 16 with 32-bit indices; with 64-bit ones,
+// which take twice the registers, 24 (FP32) and 32 (FP64) on large matrices, 16 up to 1024 blocks.
+template<typename DT, typename IT>
+bool csr_pipelined(uint64_t nrb, uint64_t rows, uint64_t nnz)
+{
+  const uint64_t line = nrb <= 512 ? 10 : sizeof(IT) == 4 || nrb <= 1024 ? 16 : sizeof(DT) == 4 ? 24 : 32;
+  return nnz / rows >= line;
+}
+
 template<typename DT, typename IT, class Epi>
 int launch_rows(hipStream_t s, const DT* val, const IT* col, const IT* rowptr, const DT* x,
-                uint64_t rows, const Epi& epi, const GridReduce& gr, const char* name)
+                uint64_t rows, uint64_t nnz, const Epi& epi, const GridReduce& gr, const char* name)
 {
   if(rows == 0) return FEAT_OK;
   const uint64_t nrb = (rows + kRowsPerBlock - 1) / kRowsPerBlock;
   const int grid = int(nrb < uint64_t(kMaxGrid) ? nrb : uint64_t(kMaxGrid));
   const GridReduce gd = reduce_for_grid(gr, uint64_t(grid));
-  // a matrix of 8-byte values that fills the chip many times over streams at the rate of a copy
-  // without the pipeline, whose loads past a block's end cost it 2 % (3D Q1 level 7, 8386
-  // row-blocks: 193 against 197 us; 4-byte values, and 5000 blocks: the pipeline, 92 against 111 us)
-  if(sizeof(DT) == 8 && nrb >= kCsrStream)
-    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 4, false>), dim3(grid), dim3(kThreads), 0, s, val, col, rowptr, x, rows, epi,
-                       gd);
+  if(csr_pipelined<DT, IT>(nrb, rows, nnz))
+    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 32 / int(sizeof(DT)), true, true>), dim3(grid), dim3(kThreads), 0, s, val,
+                       col, rowptr, x, rows, epi, gd);
+  else if(nnz / rows >= 16)
+    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 4, false, true>), dim3(grid), dim3(kThreads), 0, s, val, col, rowptr, x, rows,
+                       epi, gd);
   else
-    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 32 / int(sizeof(DT)), true>), dim3(grid), dim3(kThreads), 0, s, val, col,
-                       rowptr, x, rows, epi, gd);
+    hipLaunchKernelGGL((k_csr_rows<DT, IT, Epi, 4, false, false>), dim3(grid), dim3(kThreads), 0, s, val, col, rowptr, x, rows,
+                       epi, gd);
   finish_reduce(s, gd, uint64_t(grid));
   return check_launch(name);
 }
@@ -1246,9 +1277,9 @@ int launch_mat(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gri
   if(A->format == FEAT_FMT_CSR)
   {
     if(A->index == FEAT_IDX_U64)
-      return launch_rows<DT, uint64_t>(s, A->val, (const uint64_t*)A->col, (const uint64_t*)A->ptr, x, A->rows, epi, gr, name);
+      return launch_rows<DT, uint64_t>(s, A->val, (const uint64_t*)A->col, (const uint64_t*)A->ptr, x, A->rows, A->nnz, epi, gr, name);
     if(A->index == FEAT_IDX_U32)
-      return launch_rows<DT, uint32_t>(s, A->val, (const uint32_t*)A->col, (const uint32_t*)A->ptr, x, A->rows, epi, gr, name);
+      return launch_rows<DT, uint32_t>(s, A->val, (const uint32_t*)A->col, (const uint32_t*)A->ptr, x, A->rows, A->nnz, epi, gr, name);
   }
   else if(A->format == FEAT_FMT_SELL)
   {
@@ -2344,7 +2375,7 @@ int csr_apply_impl(feat_handle_t h, DT* r, DT a, const DT* x, DT b, const DT* y,
   {
     EpiApply<DT> e{r, y, a, b, bzero};
     GridReduce g{nullptr, nullptr, nullptr, nullptr};
-    return launch_rows<DT, IT>(h->stream, val, col, rowptr, x, rows, e, g, name);
+    return launch_rows<DT, IT>(h->stream, val, col, rowptr, x, rows, nnz, e, g, name);
   }
   // r = (b/a)*y ; r[col] += val*x[row] ; r = a*r    (arch/apply_generic.hpp:37-53)
   return feat3amd_detail::csr_apply_transposed<DT, IT>(h, r, a, x, b, bzero, y, val, col, rowptr, rows, cols, nnz, name);

@@ -1,7 +1,7 @@
-"""CSR apply against the oracle at the sizes where its pipelined passes can go wrong: row-blocks
-whose entries end on, one before and one after a pass (1024, 2048 entries), blocks
-without entries between full ones, a row over many passes, one row, and enough row-blocks for
-the streaming form (6144)."""
+"""CSR apply against the oracle at the sizes where its passes, plain or pipelined, can go wrong:
+row-blocks whose entries end on, one before and one after a pass (1024, 2048 entries), blocks
+without entries between full ones, a row over many passes, one row, many row-blocks, and the mean
+row lengths and numbers of row-blocks (512, 1024) on both sides of the lines between the forms."""
 import numpy as np
 import pytest
 
@@ -30,7 +30,30 @@ def blocks(totals):
     return lens
 
 
+def mean_rows(nblocks, mean, less=0):
+    """Ragged rows of nblocks blocks with exactly `mean` entries a row, `less` fewer in all."""
+    lens = np.random.default_rng(7).integers(0, 2 * mean + 1, nblocks * 256)
+    d = int(lens.sum()) - nblocks * 256 * mean + less
+    lens[11] += max(-d, 0)
+    for i in np.flatnonzero(lens > 1):
+        if d <= 0:
+            break
+        t = min(d, int(lens[i]) - 1)
+        lens[i] -= t
+        d -= t
+    return lens
+
+
 CASES = {
+    "pass_edges_piped": lambda: of_lengths(blocks([2047, 2048, 2049, 3071, 3072, 3073, 0, 4095, 4096, 4097, 1, 5119, 5120,
+                                                   5121, 8191, 8193, 6144, 1025, 1023, 7167]), 900),
+    "mean_10": lambda: of_lengths(mean_rows(512, 10), 4000),
+    "mean_under_10": lambda: of_lengths(mean_rows(512, 10, 1), 4000),
+    "mean_16_513": lambda: of_lengths(mean_rows(513, 16), 4000),
+    "mean_under_16_513": lambda: of_lengths(mean_rows(513, 16, 1), 4000),
+    "mean_16_1025": lambda: of_lengths(mean_rows(1025, 16), 4000),
+    "mean_24_1025": lambda: of_lengths(mean_rows(1025, 24), 4000),
+    "mean_32_1025": lambda: of_lengths(mean_rows(1025, 32), 4000),
     "one_row": lambda: of_lengths([1], 5),
     "no_entries": lambda: of_lengths([0] * 300, 7),
     "pass_edges": lambda: of_lengths(blocks([767, 768, 769, 1023, 1024, 1025, 2047, 2048, 2049, 0, 3071, 3072, 3073, 1, 0, 4097]), 900),
@@ -47,6 +70,11 @@ def test_csr_passes_bitwise(feat, handle, torch_gpu, oracle, name):
     torch = torch_gpu
     k, _ = feat.libs()
     A = CASES[name]()
+    if name == "pass_edges_piped":
+        assert A.nnz >= 10 * A.rows
+    if name.startswith("mean_"):
+        mean = int("".join(c for c in name.split("_1025")[0].split("_513")[0] if c.isdigit()))
+        assert A.nnz == mean * A.rows - ("under" in name)
     v, c, r = upload_csr(torch, A)
     rng = np.random.default_rng(9)
     x, y = rng.standard_normal(A.cols), rng.standard_normal(A.rows)
