@@ -153,6 +153,7 @@ KERNEL_API = [
     ("feat_sor_init_symbolic", _i, [_vp, C.POINTER(CsrF64), _i, C.POINTER(_vp)]),
     ("feat_sor_init_numeric", _i, [_vp, _vp, C.POINTER(CsrF64)]),
     ("feat_sor_colors", _i, [_vp, _i, C.POINTER(_i), _vp, _vp]),
+    ("feat_sor_chained", _i, [_vp, _i, C.POINTER(_i), C.POINTER(_u64)]),
     ("feat_sor_apply", _i, [_vp, _vp, _vp, _vp, _d]),
     ("feat_ssor_forward_apply", _i, [_vp, _vp, _vp, _vp, _d]),
     ("feat_ssor_backward_apply", _i, [_vp, _vp, _vp, _d]),
@@ -162,6 +163,7 @@ KERNEL_API = [
     ("feat_ilu_init_symbolic_p", _i, [_vp, C.POINTER(CsrF64), _i, C.POINTER(_vp)]),
     ("feat_ilu_apply", _i, [_vp, _vp, _vp, _vp]),
     ("feat_ilu_info", _i, [_vp, C.POINTER(_u64), C.POINTER(_u64), C.POINTER(_i), C.POINTER(_i)]),
+    ("feat_ilu_chained", _i, [_vp, _i, C.POINTER(_i), C.POINTER(_u64)]),
     ("feat_ilu_factors", _i, [_vp, _vp, _vp, _vp, _vp]),
     ("feat_ilu_done_symbolic", _i, [_vp]),
     ("feat_q1_assemble_device", _i, [_vp, _i, _i] + [_vp] * 10),
@@ -582,6 +584,12 @@ class SorPlan:
               "feat_sor_colors")
         return rank, rows[:nc.value]
 
+    def chained(self, backward=False):
+        """(whether that sweep is one launch, device bytes held for it)."""
+        on, b = _i(), _u64()
+        check(self.k.feat_sor_chained(self.s, int(backward), C.byref(on), C.byref(b)), "feat_sor_chained")
+        return bool(on.value), b.value
+
     def init_numeric(self):
         check(self.k.feat_sor_init_numeric(self.h.h, self.s, C.byref(self.desc)), "feat_sor_init_numeric")
 
@@ -622,6 +630,12 @@ class IluPlan:
 
     def init_numeric(self):
         check(self.k.feat_ilu_init_numeric(self.h.h, self.s, C.byref(self.desc)), "feat_ilu_init_numeric")
+
+    def chained(self, backward=False):
+        """(whether that solve is one launch, device bytes held for it)."""
+        on, b = _i(), _u64()
+        check(self.k.feat_ilu_chained(self.s, int(backward), C.byref(on), C.byref(b)), "feat_ilu_chained")
+        return bool(on.value), b.value
 
     def factors(self):
         l, u, d = np.empty(max(self.nnz_l, 1)), np.empty(max(self.nnz_u, 1)), np.empty(self.desc.rows)

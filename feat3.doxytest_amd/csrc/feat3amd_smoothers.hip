@@ -29,6 +29,7 @@
 #include "feat3amd_common.hpp"
 
 #include <algorithm>
+#include <new>
 #include <numeric>
 #include <utility>
 #include <vector>
@@ -122,7 +123,8 @@ __global__ void k_gather_values(uint64_t n, const uint64_t* __restrict__ map, co
 constexpr uint32_t kRing = 16384;        // positions held in LDS (128 KB)
 constexpr int kChainWaves = 16;
 constexpr uint32_t kNoRow = ~uint32_t(0);
-constexpr uint64_t kChainSlotsPerLevel = 32000;   // most entries a level of a chained sweep (see build_chain)
+constexpr uint64_t kChainFill = 16;              // most value slots of a chain for each entry of the sweep ...
+constexpr uint64_t kChainFree = uint64_t(1) << 20;   // ... beyond this many (18 MiB), see build_chain
 
 struct ChainSlice
 {
@@ -144,6 +146,7 @@ struct Chain
   uint64_t* map = nullptr;    // value slot -> source entry (kNoEntry: padding)
   uint64_t* cmap = nullptr;   // position -> source of cst
   uint64_t slots = 0;
+  uint64_t bytes = 0;         // device memory of all of it
 };
 
 template<int K>
@@ -270,34 +273,84 @@ void free_chain(Chain& c)
   c = Chain();
 }
 
+// Times of one level in microseconds: chained (`slices` slices of together `late` entries beyond
+// the K held, at most `deep` of them in a row) and as a launch of its own (rows of up to `w`
+// entries).  Fitted to ILU and SOR sweeps over 20 to 1250 levels of 64 to 7500 rows with 3 to 62
+// entries; chained / launched: 3 entries a row, 512 rows 0.6 / 2.9, 2500 rows 2.6 / 2.6, 4000
+// rows 3.9 / 2.6; 13 entries, 64 rows 0.4 / 3.5, 1500 rows 3.3 / 4.9, 2500 rows 5.7 / 4.8; 16
+// entries, 1500 rows 5.7 / 4.7; 20 entries, 512 rows 3.5 / 5.4, 1500 rows 8.2 / 5.4; 40 entries,
+// 512 rows 4.2 / 11.9.
+double chain_level_us(int K, uint64_t slices, uint64_t late, uint64_t deep)
+{
+  const double per = K == 4 ? 0.07 : 0.14;
+  return 0.3 + 0.3 * double(std::min<uint64_t>(deep, 8)) + per * (double(slices) + double(late) / 8.0);
+}
+double launch_level_us(uint64_t w) { return 2.4 + 0.14 * double(w); }
+
 // Builds the chained form of a sweep where it fits and pays; else leaves c.nslices == 0.
 //   off, perm: the level sets (rows of level l: perm[off[l] .. off[l+1])), as the per-level form
 //   begin(row), end(row), dep(k), step: the row's entries k = begin, begin + step, .. != end in
 //   sweep order, dep(k) the row entry k reads (of an earlier level); source(k) its value's index
 //   csrc(row): the index of the row's constant in its source (kNoEntry: none)
 //   pad: value of the padding entries (-0.0, or 0.0 where the kernel takes -value)
-// It fits when every level's rows and all rows they read lie within kRing positions.  It pays
-// while one workgroup runs a level in less time than a launch takes (4 to 7 us): with 13
-// entries a row 3.5 against 4.7 us on levels of 1500 rows, 5.7 against 6.4 us on 2500, and no
-// gain from 4000 on, so the line lies at kChainSlotsPerLevel entries (2500 such rows) a level.
+// It fits when every level's rows and all rows they read lie within kRing positions, and when the
+// padding (levels to 64 lanes, rows to K entries: 256 or 832 slots for a level of one row, 18
+// bytes each and half of that on the host while it is built) stays within kChainFill slots for
+// each entry or kChainFree in all: 4096 levels of one row, not a million of them at 6 or 16 KB
+// each.  It pays when the levels' times above add up to less than the launches'.  Where the memory
+// for it is not there the sweep keeps its launches as well.
 template<class Begin, class End, class Dep, class Source, class CSource>
-int build_chain(const std::vector<uint64_t>& off, const std::vector<uint32_t>& perm, int step, Begin begin, End end,
-                Dep dep, Source source, CSource csrc, double pad, Chain& c)
+int build_chain_at(const std::vector<uint64_t>& off, const std::vector<uint32_t>& perm, int step, Begin begin, End end,
+                   Dep dep, Source source, CSource csrc, double pad, Chain& c)
 {
   const size_t nl = off.size() - 1;
   const uint64_t n = perm.size();
   if(n == 0 || nl >= (size_t(1) << 31)) return FEAT_OK;
-  // rows of at most 4 entries (9-point stencils) or 13 (27-point) are held whole
-  int held = 4;
-  for(uint64_t i = 0; i < n && held == 4; ++i)
-    if((step > 0 ? end(i) - begin(i) : begin(i) - end(i)) > 4) held = 13;
+  auto length = [&](uint64_t r) { return step > 0 ? end(r) - begin(r) : begin(r) - end(r); };
+  // entries a lane holds: 4 (9-point stencils) while few of the rows are longer, else 13 (27-point)
+  uint64_t entries = 0, beyond = 0, ns = 0, need[2] = {0, 0};
+  double chained[2] = {0.0, 0.0}, launched = 0.0;
+  for(size_t l = 0; l < nl; ++l)
+  {
+    uint64_t wide = 0, late[2] = {0, 0};
+    for(uint64_t q0 = off[l]; q0 < off[l + 1]; q0 += 64, ++ns)
+    {
+      uint64_t w = 0;
+      for(uint64_t q = q0; q < std::min(q0 + 64, off[l + 1]); ++q)
+      {
+        const uint64_t len = length(perm[q]);
+        entries += len;
+        beyond += len > 4 ? len - 4 : 0;
+        w = std::max(w, len);
+      }
+      if(w > 65535) return FEAT_OK;
+      wide = std::max(wide, w);
+      for(int f = 0; f < 2; ++f)
+      {
+        const uint64_t held = f ? 13 : 4;
+        need[f] += 64 * std::max(w, held);
+        if(w > held) late[f] += w - held;
+      }
+    }
+    const uint64_t slices = (off[l + 1] - off[l] + 63) / 64;
+    for(int f = 0; f < 2; ++f)
+    {
+      const int held = f ? 13 : 4;
+      chained[f] += chain_level_us(held, slices, late[f], wide > uint64_t(held) ? wide - uint64_t(held) : 0);
+    }
+    launched += launch_level_us(wide);
+  }
+  const int pick = 4 * beyond > entries ? 1 : 0;
+  const int held = pick ? 13 : 4;
+  if(chained[pick] > launched || need[pick] > std::max(kChainFree, kChainFill * entries) ||
+     need[pick] >= (uint64_t(1) << 32) || 64 * ns >= (uint64_t(1) << 32))
+    return FEAT_OK;
   std::vector<uint32_t> pos(n);
-  uint64_t ns = 0;
+  ns = 0;
   for(size_t l = 0; l < nl; ++l)
   {
     for(uint64_t q = off[l]; q < off[l + 1]; ++q) pos[perm[q]] = uint32_t(64 * ns + (q - off[l]));
     ns += (off[l + 1] - off[l] + 63) / 64;
-    if(64 * ns >= (uint64_t(1) << 32)) return FEAT_OK;
   }
   std::vector<ChainSlice> desc;
   desc.reserve(ns);
@@ -311,10 +364,9 @@ int build_chain(const std::vector<uint64_t>& off, const std::vector<uint32_t>& p
       for(uint64_t q = q0; q < std::min(q0 + 64, off[l + 1]); ++q)
       {
         const uint64_t b = begin(perm[q]), e = end(perm[q]);
-        w = std::max<uint64_t>(w, step > 0 ? e - b : b - e);
+        w = std::max<uint64_t>(w, length(perm[q]));
         for(uint64_t k = b; k != e; k += uint64_t(std::int64_t(step))) first = std::min<uint64_t>(first, pos[dep(k)]);
       }
-      if(w > 65535) return FEAT_OK;
       desc.push_back({uint32_t(slots), uint32_t(words), uint32_t(w), uint32_t(l)});
       w = std::max<uint64_t>(w, uint64_t(held));
       slots += w;
@@ -322,7 +374,6 @@ int build_chain(const std::vector<uint64_t>& off, const std::vector<uint32_t>& p
     }
     if(first != ~uint64_t(0) && 64 * desc.size() - first > kRing) return FEAT_OK;
   }
-  if(slots >= (uint64_t(1) << 32) || 64 * slots > kChainSlotsPerLevel * nl) return FEAT_OK;
   std::vector<uint16_t> len(64 * ns, 0);
   std::vector<uint32_t> row(64 * ns, kNoRow), src(64 * words, kRing | (kRing << 16));
   std::vector<uint64_t> map(64 * slots, kNoEntry), cmap(csrc(0) == kNoEntry ? 1 : 64 * ns, kNoEntry);
@@ -353,8 +404,29 @@ int build_chain(const std::vector<uint64_t>& off, const std::vector<uint32_t>& p
   if(!rc) rc = upload(c.cmap, cmap);
   if(!rc) rc = check_hip(hipMalloc(&c.val, sizeof(double) * map.size()), "sweep plan: hipMalloc");
   if(!rc) rc = check_hip(hipMalloc(&c.cst, sizeof(double) * cmap.size()), "sweep plan: hipMalloc");
-  if(!rc) c.nslices = uint32_t(ns);
-  return rc;
+  if(rc) return rc;
+  c.nslices = uint32_t(ns);
+  c.bytes = desc.size() * sizeof(desc[0]) + len.size() * sizeof(len[0]) + row.size() * sizeof(row[0]) +
+            src.size() * sizeof(src[0]) + map.size() * (sizeof(map[0]) + sizeof(double)) +
+            cmap.size() * (sizeof(cmap[0]) + sizeof(double));
+  return FEAT_OK;
+}
+
+// build_chain_at, or no chain where its memory cannot be had
+template<class... A>
+void build_chain(Chain& c, const A&... a)
+{
+  int rc = FEAT_ERR_HIP;
+  try
+  {
+    rc = build_chain_at(a..., c);
+  }
+  catch(const std::bad_alloc&)
+  {
+  }
+  if(!rc) return;
+  free_chain(c);
+  (void)hipGetLastError();   // a failed allocation is no error of the plan's
 }
 
 // the chain's values from their sources (vals: indexed by map; consts: by cmap)
@@ -610,12 +682,10 @@ int feat_sor_init_symbolic(feat_handle_t h, const feat_csr_f64_t* A, int flags, 
   {
     auto dep = [&](uint64_t k) { return colv[k]; };
     auto same = [](uint64_t k) { return k; };
-    rc2 = build_chain(s->fw.color_off, s->fw.perm_h, 1, [&](uint64_t i) { return rp[i]; },
-                      [&](uint64_t i) { return didx[i]; }, dep, same, [&](uint64_t i) { return didx[i]; }, -0.0, s->fw.chain);
-    if(!rc2)
-      rc2 = build_chain(s->bw.color_off, s->bw.perm_h, -1, [&](uint64_t i) { return rp[i + 1] - 1; },
-                        [&](uint64_t i) { return didx[i]; }, dep, same, [&](uint64_t i) { return didx[i]; }, -0.0,
-                        s->bw.chain);
+    auto diag = [&](uint64_t i) { return didx[i]; };
+    build_chain(s->fw.chain, s->fw.color_off, s->fw.perm_h, 1, [&](uint64_t i) { return rp[i]; }, diag, dep, same, diag, -0.0);
+    build_chain(s->bw.chain, s->bw.color_off, s->bw.perm_h, -1, [&](uint64_t i) { return rp[i + 1] - 1; }, diag, dep, same,
+                diag, -0.0);
   }
   if(!rc2 && !s->fw.chain.nslices)
   {
@@ -673,6 +743,15 @@ int feat_sor_colors(feat_sor_t s, int backward, int* ncolors, uint32_t* rank_of_
   if(rank_of_row) std::copy(P.rank_of_row.begin(), P.rank_of_row.end(), rank_of_row);
   if(rows_per_color)
     for(size_t c = 0; c < nc; ++c) rows_per_color[c] = P.color_off[c + 1] - P.color_off[c];
+  return FEAT_OK;
+}
+
+int feat_sor_chained(feat_sor_t s, int backward, int* chained, uint64_t* bytes)
+{
+  if(!s) return fail(FEAT_ERR_INVALID, "feat_sor_chained: null plan");
+  const Chain& c = backward ? s->bw.chain : s->fw.chain;
+  if(chained) *chained = c.nslices != 0;
+  if(bytes) *bytes = c.bytes;
   return FEAT_OK;
 }
 
@@ -1035,11 +1114,12 @@ int feat_ilu_init_symbolic_p(feat_handle_t h, const feat_csr_f64_t* A, int p, fe
   if(!rc) rc = check_hip(hipMalloc(&s->d, sizeof(double) * (n ? n : 1)), "feat_ilu_init_symbolic: hipMalloc");
   auto same = [](uint64_t k) { return k; };
   if(!rc)
-    rc = build_chain(s->fw_off, pf, 1, [&](uint64_t i) { return rl[i]; }, [&](uint64_t i) { return rl[i + 1]; },
-                     [&](uint64_t k) { return cl[k]; }, same, [](uint64_t) { return kNoEntry; }, 0.0, s->fw);
-  if(!rc)
-    rc = build_chain(s->bw_off, pb, 1, [&](uint64_t i) { return ru[i]; }, [&](uint64_t i) { return ru[i + 1]; },
-                     [&](uint64_t k) { return cu[k]; }, same, same, 0.0, s->bw);
+  {
+    build_chain(s->fw, s->fw_off, pf, 1, [&](uint64_t i) { return rl[i]; }, [&](uint64_t i) { return rl[i + 1]; },
+                [&](uint64_t k) { return cl[k]; }, same, [](uint64_t) { return kNoEntry; }, 0.0);
+    build_chain(s->bw, s->bw_off, pb, 1, [&](uint64_t i) { return ru[i]; }, [&](uint64_t i) { return ru[i + 1]; },
+                [&](uint64_t k) { return cu[k]; }, same, same, 0.0);
+  }
   if(rc)
   {
     free_ilu(s);
@@ -1101,6 +1181,15 @@ int feat_ilu_info(feat_ilu_t s, uint64_t* nnz_l, uint64_t* nnz_u, int* levels_l,
   if(nnz_u) *nnz_u = s->nu;
   if(levels_l) *levels_l = int(s->fw_off.size() - 1);
   if(levels_u) *levels_u = int(s->bw_off.size() - 1);
+  return FEAT_OK;
+}
+
+int feat_ilu_chained(feat_ilu_t s, int backward, int* chained, uint64_t* bytes)
+{
+  if(!s) return fail(FEAT_ERR_INVALID, "feat_ilu_chained: null plan");
+  const Chain& c = backward ? s->bw : s->fw;
+  if(chained) *chained = c.nslices != 0;
+  if(bytes) *bytes = c.bytes;
   return FEAT_OK;
 }
 

@@ -887,6 +887,9 @@ int feat_sor_init_numeric(feat_handle_t h, feat_sor_t s, const feat_csr_f64_t* A
 /* the forward (backward = 0) or backward partition: number of colours, the processing rank of
  * each row's colour (n entries), rows per colour in processing order; host arrays, may be NULL */
 int feat_sor_colors(feat_sor_t s, int backward, int* ncolors, uint32_t* rank_of_row, uint64_t* rows_per_color);
+/* whether the forward (backward = 0) or backward sweep runs all its level sets in one launch, and
+ * the device memory held for that (a choice made by feat_sor_init_symbolic; same results) */
+int feat_sor_chained(feat_sor_t s, int backward, int* chained, uint64_t* bytes);
 int feat_sor_apply(feat_handle_t h, feat_sor_t s, double* y, const double* x, double omega);
 int feat_ssor_forward_apply(feat_handle_t h, feat_sor_t s, double* y, const double* x, double omega);
 int feat_ssor_backward_apply(feat_handle_t h, feat_sor_t s, double* y, double omega);
@@ -913,6 +916,8 @@ int feat_ilu_init_numeric(feat_handle_t h, feat_ilu_t s, const feat_csr_f64_t* A
 int feat_ilu_apply(feat_handle_t h, feat_ilu_t s, double* y, const double* x);
 /* entries of L and U, number of level sets of L and of U */
 int feat_ilu_info(feat_ilu_t s, uint64_t* nnz_l, uint64_t* nnz_u, int* levels_l, int* levels_u);
+/* as feat_sor_chained, for the solve with L (backward = 0) or D + U */
+int feat_ilu_chained(feat_ilu_t s, int backward, int* chained, uint64_t* bytes);
 /* copies the factors to host arrays (L and U in the order of the pattern's rows: A's lower /
  * upper entries for ILU(0), the level-p pattern's for ILU(p); the inverted diagonal); any
  * pointer may be NULL */
