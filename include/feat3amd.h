@@ -100,7 +100,7 @@ int feat_convert_u64_u32(feat_handle_t h, uint32_t* dst, const uint64_t* src, ui
  * (bit-identical to the sequential CPU loop); the transposed form computes
  * (b/a)*y, adds each column's entries in ascending entry order (the order of the
  * generic row-by-row scatter) and scales by a: bit-identical too.  The
- * transposed form takes stream-ordered buffers for the column lists (about 12 bytes per
+ * transposed form takes stream-ordered buffers for the column lists (about 16 bytes per
  * entry) from a pool of the handle's (which keeps up to 256 MiB between calls) and needs
  * nnz < 2^31; it is not for recorded graphs. */
 int feat_csr_apply_f64_u64(feat_handle_t h, double* r, double a, const double* x, double b,

@@ -1,6 +1,6 @@
 """The transposed CSR apply's column lists against the oracle, bit for bit, at the sizes where they
-can go wrong: list lengths around what one lane sorts (64) and what a workgroup holds (1024),
-dense columns, columns without entries, repeated columns in a row, unsorted rows, rows
+can go wrong: list lengths around 64, what shares a workgroup (192) and what one holds (1024),
+many long columns, lists whose parts by entry number do not fit (clustered entries), dense columns, columns without entries, repeated columns in a row, unsorted rows, rows
 without entries, tiles of entries that start and end inside a row."""
 import numpy as np
 import pytest
@@ -22,7 +22,22 @@ def by_columns(rng, rows, lens):
     return Csr(rows, len(lens), rng.standard_normal(col.size), col[order].astype(np.uint64), rp)
 
 
+def clustered(rng):
+    """Column 0: 3000 entries in a row, and one far behind them; column 1: 5000 spread evenly."""
+    mid = np.concatenate([rng.integers(2, 300, 60000), np.full(5000, 1)])
+    rng.shuffle(mid)
+    col = np.concatenate([np.zeros(3000, np.int64), mid, [0]])
+    rp = np.concatenate([[0], np.sort(rng.integers(0, col.size, 199)), [col.size]]).astype(np.uint64)
+    return Csr(200, 300, rng.standard_normal(col.size), col.astype(np.uint64), rp)
+
+
 CASES = {
+    "clustered": clustered,
+    "around_192": lambda g: by_columns(g, 700, [191, 192, 193, 194, 0, 190] * 9),
+    "few_columns": lambda g: by_columns(g, 700, [192, 193, 1, 100, 64]),
+    "many_long": lambda g: by_columns(g, 3000, [2900] * 70),
+    "many_medium": lambda g: by_columns(g, 3000, [65, 70, 200] * 500),
+    "long_steps": lambda g: by_columns(g, 9000, [1025, 2047, 3, 4097, 0, 8193, 1026] * 3),
     "one": lambda g: by_columns(g, 1, [1]),
     "short": lambda g: by_columns(g, 500, [0, 1, 2, 63, 64] * 40),
     "around_64": lambda g: by_columns(g, 300, [63, 64, 65, 66, 127, 128, 129] * 19),
