@@ -34,7 +34,10 @@
 // the name is only a stand-in for the symbol): it uses the per-device address that
 // hipGetSymbolAddress returned at handle creation.  Every call on one GPU shares that
 // GPU's copy, so calls that overlap on one GPU race; nothing in it needs to start at zero.
-static __device__ __align__(256) unsigned char scratch[FEAT_TR_NOALLOC_SCRATCH_BYTES];
+// Beyond the documented size it holds what does not grow with the entries: the scan's sums (4
+// bytes for each kTrScan columns) and the alignment of the parts.
+constexpr size_t kTrScratchSlack = size_t(64) << 10;
+static __device__ __align__(256) unsigned char scratch[FEAT_TR_NOALLOC_SCRATCH_BYTES + kTrScratchSlack];
 
 namespace {
 
@@ -605,7 +608,7 @@ int csr_apply_transposed_noalloc(feat_handle_t h, DT* r, DT a, const DT* x, DT b
     return fail(FEAT_ERR_UNSUPPORTED, "csr_apply_transposed_noalloc: the matrix needs more than the 32 MiB scratch "
                                       "(20 bytes per entry and 4 per column)");
   const TrLayout L(cols, nnz);
-  if(L.bytes > kTrScratchBytes)
+  if(L.bytes > kTrScratchBytes + kTrScratchSlack)
     return fail(FEAT_ERR_UNSUPPORTED, "csr_apply_transposed_noalloc: the matrix needs more than the 32 MiB scratch");
   return tr_apply(h->stream, base, L, r, a, x, b, bzero, y, val, col, rowptr, rows, cols, nnz, name);
 }

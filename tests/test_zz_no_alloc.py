@@ -12,6 +12,7 @@ from tests.test_gpu_lafem import dev, host, upload_csr
 pytestmark = pytest.mark.gpu
 
 FEAT_ERR_UNSUPPORTED = 5
+FEAT_TR_BYTES = 32 << 20   # FEAT_TR_NOALLOC_SCRATCH_BYTES
 
 
 def _both(feat, handle, torch, A, x, y, a, b):
@@ -64,3 +65,26 @@ def test_noalloc_transposed_rejects_oversize(feat, handle, torch_gpu):
     assert b"32 MiB" in k.feat_last_error()
     torch.cuda.synchronize()
     assert torch.all(r == 3.0)
+
+
+@pytest.mark.parametrize("cols,nnz", [(8388607, 0), (8388000, 100), (8300000, 17000), (0, 1677721)])
+def test_noalloc_transposed_takes_its_limit(feat, handle, torch_gpu, cols, nnz):
+    """Every matrix within 20 bytes an entry and 4 a column of the scratch is taken, many columns too."""
+    torch = torch_gpu
+    k, _ = feat.libs()
+    cols = cols or (FEAT_TR_BYTES - 20 * nnz) // 4
+    assert 20 * nnz + 4 * cols <= FEAT_TR_BYTES
+    rows = 50
+    g = torch.Generator(device="cuda").manual_seed(nnz)
+    rp = torch.linspace(0, nnz, rows + 1, device="cuda").long()
+    rp[-1] = nnz
+    col = torch.randint(0, cols, (max(nnz, 1),), generator=g, device="cuda")
+    val = torch.ones(max(nnz, 1), dtype=torch.float64, device="cuda")
+    x = torch.ones(rows, dtype=torch.float64, device="cuda")
+    y = torch.full((cols,), 2.0, dtype=torch.float64, device="cuda")
+    r = torch.full((cols,), 3.0, dtype=torch.float64, device="cuda")
+    feat.check(k.feat_csr_apply_transposed_noalloc_f64_u64(handle.h, feat.ptr(r), 1.0, feat.ptr(x), 0.5, feat.ptr(y),
+                                                           feat.ptr(val), feat.ptr(col), feat.ptr(rp), rows, cols, nnz), "noalloc")
+    want = 1.0 + torch.bincount(col[:nnz], minlength=cols).double()   # whole numbers: any order
+    torch.cuda.synchronize()
+    assert torch.equal(r, want)
