@@ -695,6 +695,7 @@ constexpr int kMaxTrip = 10;
 constexpr uint32_t kDiagNone = 255u;   // slot without an entry
 // uniform-stencil march: from this many one-plane workgroups on, a lane takes three planes
 constexpr uint64_t kSten3 = 1024;
+constexpr uint64_t kStenOne = 8192;   // see k_sten_rows
 
 // SpMV-type row loop over the diagonal plan: the slots run in ascending offset order (=
 // ascending columns, the CSR order), each lane adds its entry of a slot if it has one.
@@ -817,9 +818,9 @@ __global__ __launch_bounds__(kThreads) void k_sell_diag_rows(const DT* __restric
 // rows they belong to are boundary rows.  A boundary row that the epilogue filters does not
 // use its sum and is finished in place; the others are summed from their codes at the end, one
 // lane per boundary row.  Those rows come after the march, with scattered loads of their own, and
-// cost a small 3D grid more than the march gains: sten_marches.  Nine loads at a time (one at a
+// cost a small 3D grid more than the march gains: sten_marches.  Nine loads at a time: one at a
 // time, each behind its code's branch, a smoother call of 4 steps with no filter took 67 us instead of
-// 51 on 97^3 nodes in FP64, 28 instead of 25 on 513^2; 91 instead of 97 on 129^3).
+// 51 on 97^3 nodes in FP64, 28 instead of 25 on 513^2.
 __host__ __device__ inline uint32_t grid_boundary_rows(int dim, uint32_t n1)
 {
   return dim == 3 ? 2 * n1 * n1 + (n1 - 2) * (4 * n1 - 4) : 4 * n1 - 4;
@@ -850,9 +851,11 @@ __host__ __device__ constexpr size_t sten_offset()
   return (256 * sizeof(DT) + (256 + 1 + kMaxTrip) * sizeof(int) + 7) & ~size_t(7);
 }
 
-// CLOSED (the caller's hint that there are no such rows): one load at a time, in the smaller kernel
-// (the solves' steps on coarse levels 3.96 us instead of 4.10).
-template<typename DT, class Epi, int DIM, int ZC, bool CLOSED>
+// ONE: one load at a time.  That kernel is the smaller one (the solves' steps on coarse levels 3.96 us
+// instead of 4.10), so it serves the callers that have filtered the boundary; and with many
+// workgroups other waves hide its loads, of which it issues fewer (a call of 4 steps with no
+// filter, one / nine at a time: 113^3 nodes 77 / 71 us, 129^3 91 / 97 us): launch_sten.
+template<typename DT, class Epi, int DIM, int ZC, bool ONE>
 __global__ __launch_bounds__(kThreads) void k_sten_rows(const DT* __restrict__ tab, const uint32_t* __restrict__ codes,
                                                         int n1, const DT* __restrict__ x, uint32_t rows, Epi epi,
                                                         GridReduce gr)
@@ -935,7 +938,7 @@ __global__ __launch_bounds__(kThreads) void k_sten_rows(const DT* __restrict__ t
     const uint32_t* cw = codes + uint64_t(row >> 6) * 64 * NW + (row & 63);
     auto place = [&](int t) { return t % 3 - 1 + (DIM == 3 ? (t / 3) % 3 - 1 : t / 3 - 1) * m + (DIM == 3 ? t / 9 - 1 : 0) * P; };
     DT sum = DT(0);
-    if constexpr(CLOSED)
+    if constexpr(ONE)
     {
 #pragma unroll
       for(int t = 0; t < 3 * NT; ++t)
@@ -987,7 +990,7 @@ __global__ __launch_bounds__(kThreads) void k_sten_rows(const DT* __restrict__ t
 // smaller grids keep the code words otherwise, as the mask may leave boundary rows to sum.  A
 // smoother call of 4 steps in FP64, code words / march: 33^3 nodes filtered 18 / 18 us, open
 // 17 / 28; 65^3 filtered 28 / 27, open 26 / 37; 97^3 filtered 64 / 51, open 58 / 51; 129^3
-// filtered 121 / 83, open 109 / 97.  2D, 513^2 filtered 26 / 22, open 26 / 25.
+// filtered 121 / 83, open 109 / 91.  2D, 513^2 filtered 26 / 22, open 26 / 25.
 constexpr uint64_t kStenOpen = 3584;
 template<class M>
 bool sten_marches(const M* A)
@@ -1003,12 +1006,12 @@ int launch_sten(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gr
 {
   const uint32_t n1 = A->grid_n1, dim = A->grid_dim;
   const uint32_t P = dim == 3 ? n1 * n1 : n1, ngrp = (P + kHaloChunk - 1) / kHaloChunk;
-  auto go = [&](auto zc, auto d, auto closed) {
+  auto go = [&](auto zc, auto d, auto by_one) {
     constexpr int ZC = decltype(zc)::value, DIM = decltype(d)::value;
     const uint64_t items = uint64_t(ngrp) * ((n1 + ZC - 1) / ZC);
     const int grid = int(items < uint64_t(kMaxGrid) ? items : uint64_t(kMaxGrid));
     const GridReduce gd = reduce_for_grid(gr, uint64_t(grid));
-    hipLaunchKernelGGL((k_sten_rows<DT, Epi, DIM, ZC, decltype(closed)::value>), dim3(grid), dim3(kThreads), 0, s,
+    hipLaunchKernelGGL((k_sten_rows<DT, Epi, DIM, ZC, decltype(by_one)::value>), dim3(grid), dim3(kThreads), 0, s,
                        reinterpret_cast<const DT*>(A->val), static_cast<const uint32_t*>(A->col), int(n1), x,
                        uint32_t(A->rows), epi, gd);
     finish_reduce(s, gd, uint64_t(grid));
@@ -1020,8 +1023,9 @@ int launch_sten(hipStream_t s, const M* A, const DT* x, const Epi& epi, const Gr
   using two_d = integral_constant<int, 2>;
   using yes = std::true_type;
   using no = std::false_type;
-  const bool many = uint64_t(ngrp) * n1 >= kSten3;   // workgroups with one plane a lane
-  if(dim == 3 && !A->grid_closed) return go(three(), three(), no());   // at least kStenOpen of them (sten_marches)
+  const uint64_t wg1 = uint64_t(ngrp) * n1;   // workgroups with one plane a lane
+  const bool many = wg1 >= kSten3;
+  if(dim == 3 && !A->grid_closed && wg1 < kStenOne) return go(three(), three(), no());   // >= kStenOpen (sten_marches)
   if(dim == 3) return many ? go(three(), three(), yes()) : go(one(), three(), yes());
   if(A->grid_closed) return many ? go(three(), two_d(), yes()) : go(one(), two_d(), yes());
   return many ? go(three(), two_d(), no()) : go(one(), two_d(), no());
