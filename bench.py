@@ -950,10 +950,10 @@ def main():
                                     "the transfer operators in FP16 and uses the FP32 dictionary elsewhere",
                             "variable_coefficient_level7": mixed_vc},
         "spmv": {
-            "sell64_diag": {"kernel": "k_sten_rows<double,EpiApply<double>,3,3>", "us_per_launch": dict_ms * 1e3,
+            "sell64_diag": {"kernel": "k_sten_rows<double,EpiApply<double>,3,3,true>", "us_per_launch": dict_ms * 1e3,
                             "bytes_per_launch": dict_bytes, "gbps": dict_gbs,
                             "csr_equivalent_gbps": csr_bytes / (dict_ms * 1e-3) / 1e9,
-                     "jacobi_step": {"kernel": "k_sten_rows<double,EpiSmooth<double>,3,3> (one fused "
+                     "jacobi_step": {"kernel": "k_sten_rows<double,EpiSmooth<double>,3,3,true> (one fused "
                                                "Richardson(Jacobi) step, the solve's most frequent launch)",
                                      "us_per_launch": step_ms * 1e3, "achieved": step_gbs,
                                      "frac": step_gbs / PEAK_HBM_GBS, "algorithmic_bytes": step_bytes}, "stored_slots": dict_padded},
@@ -976,7 +976,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
                      "frac": achieved / PEAK_HBM_GBS, "traffic": SPMV_TRAFFIC_BYTES["jacobi_step"],
                      "algorithmic_bytes": step_bytes, "us_per_launch": step_ms * 1e3,
-                     "kernel": "k_sten_rows<double,EpiSmooth<double>,3,3>: one fused Richardson(Jacobi) "
+                     "kernel": "k_sten_rows<double,EpiSmooth<double>,3,3,true>: one fused Richardson(Jacobi) "
                                "step x_{k+1} = x_k + 0.5 filter(inv_diag (rhs - A x_k)) on the level-7 diagonal "
                                "pair-dictionary plan with uniform interior rows (the solve's dominant kernel: 35 "
                                "of its launches per solve), bytes = stencil + code words of the boundary rows + "

@@ -4,9 +4,10 @@
 //  * CSR SpMV: rows are processed in row-blocks of kRowsPerBlock (256, one lane
 //    per row).  A 256-thread workgroup streams the contiguous nonzero range of its
 //    row-block through LDS in passes of 1024 or 2048 entries (val and the gathered
-//    x[col] side by side, fully coalesced 64-wide loads, two passes ahead), and
-//    each lane sums its row's entries from LDS in storage order with one fma per
-//    entry.  The per-row arithmetic is therefore exactly the
+//    x[col] side by side, fully coalesced 64-wide loads; two passes ahead where
+//    the rows are long enough, see csr_pipelined), and each lane sums its row's
+//    entries from LDS in storage order with one fma per entry.  The per-row
+//    arithmetic is therefore exactly the
 //    reference's sequential loop (arch/apply_generic.hpp:57-66), bit for bit,
 //    while HBM sees only coalesced streams.  Fused epilogues apply the unit
 //    filter (bit mask), the defect/Richardson/Jacobi updates and reductions.
@@ -1154,9 +1155,11 @@ __global__ __launch_bounds__(kThreads) void k_dlinear_rows(int dim, int n1, cons
 // negative offset is the entry of row i + offset at the opposite slot, so only the slots from
 // the diagonal on are streamed, 14 of 27, and the others are read where the rows below have just
 // brought them into the XCD's L2 (consecutive chunks run on one XCD).  The value arrays go
-// through the caches then.  A smoother call of 4 steps on 129^3 nodes: FP64 461 -> 337 us
-// (3.7 TB/s of the bytes left), FP32 215 -> 115 us (5.4 TB/s), FP16 values 150 -> 100 us; on
-// 65^3 nodes 72 -> 52, 34 -> 28, 31 -> 27 us.  Marching over planes as k_sten_rows does (3 loads
+// through the caches then.  A smoother call of 4 steps, the same symmetric values through all slots
+// and through 14: 129^3 nodes FP64 447 -> 330 us (3.7 TB/s of the bytes left), FP32 211 -> 100 us,
+// FP16 values 140 -> 86 us; 65^3 nodes 66 -> 47, 32 -> 25, 27 -> 25 us.  2D (5 of 9 slots): 1025^2
+// nodes 88 -> 58, 46 -> 34, 37 -> 31 us, 513^2 29 -> 26, 18 and 17 either way, 257^2 and smaller
+// 15 to 16 either way.  Values that differ in one bit keep all slots.  Marching over planes as k_sten_rows does (3 loads
 // of x a row instead of 27) gained nothing here and cost 20 to 50 % on 65^3 nodes.
 template<typename DT, typename VT, class Epi, int DIM, bool SYM>
 __global__ __launch_bounds__(kThreads) void k_band_rows(const VT* __restrict__ val, int n1,
@@ -1185,7 +1188,8 @@ __global__ __launch_bounds__(kThreads) void k_band_rows(const VT* __restrict__ v
     // unconditionally (each slot array spans all rows, and an outside neighbour reads x[i];
     // both are left out of the sum), since a predicated 16-bit load is compiled into a
     // branch that waits for it before converting (FP16 plan 1.8x slower).  Wider values
-    // keep predicated loads, which measured faster for them (FP64 solve 70.4 against 78.9 ms).
+    // keep predicated loads, which measured faster for them (level-7 FP64 solve with all slots
+    // 70.4 against 78.9 ms).
     VT v[NS];
     DT xv[NS];
 #pragma unroll
@@ -3753,7 +3757,7 @@ constexpr int kTailSmoothed = FEAT_MG_TAIL_MAX_LEVELS - 1;
 //    row's 3^dim values stay in registers for the 4 or 5 sweeps of a leg, so a leg reads them
 //    once from the caches, and only for free rows; a kernel per dimension keeps them out of
 //    scratch (with the dimension at run time a third of them went there: 63 us instead of 37).
-//    729 + 125 rows over a direct 27, V(4,4): 37 us in FP64, 30 us in FP32 with FP16 values,
+//    729 + 125 rows over a direct 27, V(4,4): 38 us in FP64, 31 us in FP32 with FP16 values,
 //    against about 100 us of 25 launches.
 enum TailMode { kTailPlan, kTailGrid, kTailBand2, kTailBand3 };
 template<typename DT, int MODE>
